@@ -462,7 +462,7 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
             for (int a = 0; a < 3; a++) d[a] = X.sub(FV[lp.a][12 + a], FV[lp.b][12 + a]);
             V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
             X.os << "        work += " << kSelf << "u;\n";
-            X.os << "        if (__ballot(" << X.ref(d2) << " < " << lit(cull) << ")) {\n";
+            X.os << "        if (__ballot(" << X.ref(d2) << " < " << lit(cull) << ")" << (cost ? "" : " & live") << ") {\n";
             int nsp = (int)(A.spheres.size() + B.spheres.size());
             X.os << "            work += " << (int)lp.pairs.size() * kSelf + nsp * kXform << "u;\n";
             if (!cost) {
@@ -489,28 +489,37 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                         X.os << "            h |= " << X.ref(dd) << " < " << lit(std::min(thr, sqrt_threshold(sr))) << ";\n";
                     }
                 }
-                X.os << "        }\n        }\n";
-                X.os << "        if (mp_stop<MODE>(h, mask)) return h;\n        }\n";
+                X.os << "            const u64 hb = __ballot(h);\n"
+                        "            if (mp_decides<MODE>(hb, mask)) return h;\n"
+                        "            live = mp_live<MODE>(hb, mask);\n"
+                        "        }\n        }\n        }\n";
                 continue;
             }
             std::map<int, std::array<V, 3>> cs;
             for (int s : A.spheres) { V c[3]; centre(X, s, c); cs[s] = {c[0], c[1], c[2]}; }
             for (int s : B.spheres) { V c[3]; centre(X, s, c); cs[s] = {c[0], c[1], c[2]}; }
-            for (auto& pr : lp.pairs) {
-                int i = pr.first, j = pr.second;
-                float thr, sr;
-                pair_thr(i, j, thr, sr);
-                V e[3];
-                for (int a = 0; a < 3; a++) e[a] = X.sub(cs[i][a], cs[j][a]);
-                V dd = X.dot3(e[0], e[0], e[1], e[1], e[2], e[2]);
-                if (cost)
-                    X.os << "            part += " << X.ref(dd) << " < " << lit(thr) << " ? " << lit(sr) << " - __builtin_sqrtf("
-                         << X.ref(dd) << ") : 0.0f;\n";
-                else
-                    X.os << "            h |= " << X.ref(dd) << " < " << lit(std::min(thr, sqrt_threshold(sr))) << ";\n";
+            // the pairs of one sphere of A at a time: its distances first, the penetrations (a correctly
+            // rounded square root each) only when some lane has a contact among them; a pair without
+            // one adds an exact zero
+            for (size_t p0 = 0; p0 < lp.pairs.size(); p0 += B.spheres.size()) {
+                std::string any;
+                std::vector<std::string> terms;
+                for (size_t p = p0; p < p0 + B.spheres.size(); p++) {
+                    int i = lp.pairs[p].first, j = lp.pairs[p].second;
+                    float thr, sr;
+                    pair_thr(i, j, thr, sr);
+                    V e[3];
+                    for (int a = 0; a < 3; a++) e[a] = X.sub(cs[i][a], cs[j][a]);
+                    V dd = X.dot3(e[0], e[0], e[1], e[1], e[2], e[2]);
+                    const std::string c = X.ref(dd) + " < " + lit(thr);
+                    any += (any.empty() ? "" : " | ") + ("(" + c + ")");
+                    terms.push_back("                part += " + c + " ? " + lit(sr) + " - __builtin_sqrtf(" + X.ref(dd) + ") : 0.0f;\n");
+                }
+                X.os << "            if (__ballot(" << any << ")) {\n";
+                for (const std::string& t : terms) X.os << t;
+                X.os << "            }\n";
             }
             X.os << "        }\n        }\n";
-            if (!cost) X.os << "        if (mp_stop<MODE>(h, mask)) return h;\n        }\n";
         }
         return X.os.str();
     };
@@ -546,8 +555,9 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
             } else {
                 V d[3] = {GP.sub(FV[k][12], c[0]), GP.sub(FV[k][13], c[1]), GP.sub(FV[k][14], c[2])};
                 V dd = GP.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
-                V sq = dd.k ? K(std::sqrt(dd.c)) : GP.tmp("__builtin_sqrtf(" + GP.ref(dd) + ")");
-                term = GP.add(sq, K(Rk));
+                // a cull's radius: the hardware square root, rounded up by 1e-6 relative
+                term = dd.k ? K(std::sqrt(dd.c) * 1.000001f + Rk)
+                            : GP.tmp("__builtin_fmaf(__builtin_amdgcn_sqrtf(" + GP.ref(dd) + "), 1.000001f, " + lit(Rk) + ")");
             }
             if (first) {
                 r = term;
@@ -561,6 +571,26 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
         gsph.push_back({c[0], c[1], c[2], r});
     }
     const std::string group_prologue = GP.os.str();
+    const int G = (int)groups.size();
+    // the groups' balls over the wave's live states (mp_half_balls), and the near obstacles of the
+    // chunk of 64 from `base` on
+    std::string group_balls, group_near = "            const float reach = mp_bound_reach(ob);\n", near_any;
+    for (int gi = 0; gi < G; gi++) {
+        const std::string g = std::to_string(gi);
+        group_balls += "        const HalfBalls hb" + g + " = mp_half_balls(" + GP.ref(gsph[gi][0]) + ", " + GP.ref(gsph[gi][1]) +
+                       ", " + GP.ref(gsph[gi][2]) + ", " + GP.ref(gsph[gi][3]) + ", live);\n";
+        group_near += "            const u64 gm" + g + " = mp_near(ob, reach, hb" + g + ", seen);\n";
+        near_any += (gi ? " | gm" : "gm") + g;
+    }
+    if (G == 0) near_any = "0ull";
+    // The link frames made opaque at the head of each near obstacle's block: otherwise the sphere
+    // centres, which do not change from obstacle to obstacle, are moved out of the loop, far more of
+    // them than there are registers (FR3's check kernel 258 -> 212 VGPRs, two waves per SIMD again;
+    // mp_plan 383 -> 308)
+    std::string pin;
+    for (int k = 0; k < NL; k++)
+        for (int e = 0; e < 15; e++)
+            if (!FV[k][e].k) pin += "            asm volatile(\"\" : \"+v\"(" + FV[k][e].e + "));\n";
 
     // ---------------------------------------------------------------- environment blocks
     // kind: 0 box, 1 sphere, 2 capsule, 3 cylinder.  The obstacle parameters are named
@@ -574,26 +604,17 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
         const V oc[3] = {V{false, 0.0f, kind == 1 ? "ox" : "ocx"}, V{false, 0.0f, kind == 1 ? "oy" : "ocy"},
                          V{false, 0.0f, kind == 1 ? "oz" : "ocz"}};
         const std::string orr = kind == 1 ? "orad" : "orr";
-        const bool cull_group = groups.size() > 1;
-        // all group tests of this obstacle first (straight-line code, no branch in between), then
-        // one branch for the common case that no lane is near any group
-        if (cull_group) {
-            std::string any;
-            for (size_t gi = 0; gi < groups.size(); gi++) {
-                V gd[3] = {X.sub(gsph[gi][0], oc[0]), X.sub(gsph[gi][1], oc[1]), X.sub(gsph[gi][2], oc[2])};
-                V gd2 = X.dot3(gd[0], gd[0], gd[1], gd[1], gd[2], gd[2]);
-                V gs = X.tmp(X.ref(gsph[gi][3]) + " + " + orr);
-                X.os << "            const u64 gb" << gi << " = __ballot(" << X.ref(gd2) << " < " << X.ref(gs) << " * "
-                     << X.ref(gs) << ");\n";
-                any += (gi ? " | gb" : "gb") + std::to_string(gi);
-            }
-            X.os << "            work += " << kSph * (int)groups.size() << "u;\n";
-            X.os << "            if (" << any << ") {\n" << detail;
-        } else {
-            X.os << detail;
+        X.os << pin << detail;
+        for (int gi = 0; gi < G; gi++) {
+        // the groups whose ball the obstacle reaches, then those with a live state near it
+        X.os << "            if ((gm" << gi << " >> l) & 1ull) {\n";
+        {
+            V gd[3] = {X.sub(gsph[gi][0], oc[0]), X.sub(gsph[gi][1], oc[1]), X.sub(gsph[gi][2], oc[2])};
+            V gd2 = X.dot3(gd[0], gd[0], gd[1], gd[1], gd[2], gd[2]);
+            V gs = X.tmp(X.ref(gsph[gi][3]) + " + " + orr);
+            X.os << "            work += " << kSph << "u;\n";
+            X.os << "            if (__ballot(" << X.ref(gd2) << " < " << X.ref(gs) << " * " << X.ref(gs) << ") & live) {\n";
         }
-        for (size_t gi = 0; gi < groups.size(); gi++) {
-        if (cull_group) X.os << "            {\n            if (gb" << gi << ") {\n";
         for (int k : groups[gi]) {
             const SphereLink& L = SL[k];
             float Rm = (float)(L.R + kCullMargin);
@@ -614,8 +635,7 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                     V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
                     cond = X.ref(d2) + " < " + lit(Rm * Rm);
                 } else {
-                    V sdf = X.tmp("mp_cyl_sdf(" + X.ref(l[0]) + ", " + X.ref(l[1]) + ", " + X.ref(l[2]) + ", crad, hh)");
-                    cond = X.ref(sdf) + " < " + lit(Rm);
+                    cond = "mp_cyl_near(" + X.ref(l[0]) + ", " + X.ref(l[1]) + ", " + X.ref(l[2]) + ", crad, hh, " + lit(Rm) + ")";
                 }
             } else if (kind == 1) {
                 V d[3] = {X.sub(b[0], V{false, 0, "ox"}), X.sub(b[1], V{false, 0, "oy"}), X.sub(b[2], V{false, 0, "oz"})};
@@ -628,7 +648,7 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                 cond = X.ref(d2) + " < " + X.ref(sr) + " * " + X.ref(sr);
             }
             X.os << "            work += " << tcost << "u;\n";
-            X.os << "            if (__ballot(" << cond << ")) {\n";
+            X.os << "            if (__ballot(" << cond << ") & live) {\n";
             X.os << "                work += " << n * (kXform + tcost) << "u;\n";
             // spheres and capsules: contact <=> d2 < (r+R)^2 and sqrtf(d2) < r+R (the cost
             // (r+R) - sqrtf(d2) is then > 0); a fast test with a 1e-6 relative margin, then the
@@ -650,8 +670,9 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                         d[a] = X.tmp(X.ref(l[a]) + " - fminf(fmaxf(" + X.ref(l[a]) + ", " + lo[a] + "), " + hi[a] + ")");
                     V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
                     if (cost)
-                        X.os << "                part += " << X.ref(d2) << " < " << lit(r * r) << " ? " << lit(r)
-                             << " - __builtin_sqrtf(" << X.ref(d2) << ") : 0.0f;\n";
+                        X.os << "                if (__ballot(" << X.ref(d2) << " < " << lit(r * r) << "))\n                    part += "
+                             << X.ref(d2) << " < " << lit(r * r) << " ? " << lit(r) << " - __builtin_sqrtf(" << X.ref(d2)
+                             << ") : 0.0f;\n";
                     else
                         X.os << "                hit |= " << X.ref(d2) << " < " << lit(boxte[s]) << ";\n";
                 } else if (kind == 1) {
@@ -659,7 +680,8 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                     V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
                     V sr = X.tmp(lit(r) + " + orad");
                     if (cost) {
-                        X.os << "                part += " << X.ref(d2) << " < " << X.ref(sr) << " * " << X.ref(sr)
+                        X.os << "                if (__ballot(" << X.ref(d2) << " < " << X.ref(sr) << " * " << X.ref(sr)
+                             << "))\n                    part += " << X.ref(d2) << " < " << X.ref(sr) << " * " << X.ref(sr)
                              << " ? fmaxf(0.0f, " << X.ref(sr) << " - __builtin_sqrtf(" << X.ref(d2) << ")) : 0.0f;\n";
                     } else {
                         V T2 = X.tmp(X.ref(sr) + " * " + X.ref(sr));
@@ -672,7 +694,8 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                     V d2 = X.tmp("mp_cap_d2(" + X.ref(c[0]) + ", " + X.ref(c[1]) + ", " + X.ref(c[2]) + ", x1, y1, z1, xv, yv, zv, rdv)");
                     V rs = X.tmp(lit(r) + " + crad");
                     if (cost) {
-                        X.os << "                part += " << X.ref(d2) << " < " << X.ref(rs) << " * " << X.ref(rs)
+                        X.os << "                if (__ballot(" << X.ref(d2) << " < " << X.ref(rs) << " * " << X.ref(rs)
+                             << "))\n                    part += " << X.ref(d2) << " < " << X.ref(rs) << " * " << X.ref(rs)
                              << " ? fmaxf(0.0f, " << X.ref(rs) << " - __builtin_sqrtf(" << X.ref(d2) << ")) : 0.0f;\n";
                     } else {
                         V T2 = X.tmp(X.ref(rs) + " * " + X.ref(rs));
@@ -684,12 +707,15 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                 } else {
                     V l[3];
                     for (int a = 0; a < 3; a++) l[a] = X.row(mm[4 * a], c[0], mm[4 * a + 1], c[1], mm[4 * a + 2], c[2], mm[4 * a + 3]);
+                    // the distance takes two square roots: only when some lane's sphere is near
+                    X.os << "                if (__ballot(mp_cyl_near(" << X.ref(l[0]) << ", " << X.ref(l[1]) << ", " << X.ref(l[2])
+                         << ", crad, hh, " << lit(r) << "))" << (cost ? "" : " & live") << ") {\n";
                     V sdf = X.tmp("mp_cyl_sdf(" + X.ref(l[0]) + ", " + X.ref(l[1]) + ", " + X.ref(l[2]) + ", crad, hh)");
                     if (cost)
-                        X.os << "                { const float pen = " << lit(r) << " - " << X.ref(sdf)
+                        X.os << "                const float pen = " << lit(r) << " - " << X.ref(sdf)
                              << "; part += pen > 0.0f ? pen : 0.0f; }\n";
                     else
-                        X.os << "                hit |= " << X.ref(sdf) << " < " << lit(r) << ";\n";
+                        X.os << "                hit |= " << X.ref(sdf) << " < " << lit(r) << "; }\n";
                 }
             }
             if (banded) {
@@ -701,9 +727,8 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
             }
             X.os << "            }\n            }\n";
         }
-        if (cull_group) X.os << "            }\n            }\n";
+        X.os << "            }\n            }\n";
         }
-        if (cull_group) X.os << "            }\n";
         return X.os.str();
     };
 
@@ -727,69 +752,90 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
          "        float* row = tile + lane * MP_CENTRE_ROW;\n"
       << staged_body << "    }\n";
     o << "    template <int MODE>\n    static __device__ __forceinline__ bool self_hit(const float* F, bool h, u64 mask, unsigned& work, const Team& T) {\n"
+         "        u64 live = mp_live<MODE>(__ballot(h), mask);\n"
       << self_body(false) << "        return h;\n    }\n";
     o << "    static __device__ __forceinline__ float self_cost(const float* F, unsigned& work) {\n        float part = 0.0f;\n"
       << self_body(true) << "        return part;\n    }\n";
-    // an obstacle's bounding sphere first (its own section of the scene), its record only when a
-    // link group is near it
-    const char* box_load =
-        "            const float* bb = sc.bbox + o * 4;\n"
-        "            const float ocx = mp_sld(bb + 0), ocy = mp_sld(bb + 1), ocz = mp_sld(bb + 2), orr = mp_sld(bb + 3);\n";
+    // a near obstacle's bounding sphere comes from the lane that tested it, its record by scalar loads
+    const char* bound_load =
+        "            const float ocx = mp_lane(ob.x, l), ocy = mp_lane(ob.y, l), ocz = mp_lane(ob.z, l), orr = mp_lane(ob.w, l);\n";
+    const char* sph_load =
+        "            const float ox = mp_lane(ob.x, l), oy = mp_lane(ob.y, l), oz = mp_lane(ob.z, l), orad = mp_lane(ob.w, l);\n";
     const char* box_detail =
-        "            const float* b = sc.box + o * MP_BOX_W;\n"
+        "            const float* b = sc.box + k * MP_BOX_W;\n"
         "            const float m0 = mp_sld(b + 0), m1 = mp_sld(b + 1), m2 = mp_sld(b + 2), m3 = mp_sld(b + 3);\n"
         "            const float m4 = mp_sld(b + 4), m5 = mp_sld(b + 5), m6 = mp_sld(b + 6), m7 = mp_sld(b + 7);\n"
         "            const float m8 = mp_sld(b + 8), m9 = mp_sld(b + 9), m10 = mp_sld(b + 10), m11 = mp_sld(b + 11);\n"
         "            const float lox = mp_sld(b + 12), loy = mp_sld(b + 13), loz = mp_sld(b + 14);\n"
         "            const float hix = mp_sld(b + 15), hiy = mp_sld(b + 16), hiz = mp_sld(b + 17);\n";
-    const char* sph_load =
-        "            const float* p = sc.sph + o * MP_SPH_W;\n"
-        "            const float ox = mp_sld(p + 0), oy = mp_sld(p + 1), oz = mp_sld(p + 2), orad = mp_sld(p + 3);\n";
-    const char* cap_load =
-        "            const float* kb = sc.bcap + o * 4;\n"
-        "            const float ocx = mp_sld(kb + 0), ocy = mp_sld(kb + 1), ocz = mp_sld(kb + 2), orr = mp_sld(kb + 3);\n";
     const char* cap_detail =
-        "            const float* k = sc.cap + o * MP_CAP_W;\n"
-        "            const float x1 = mp_sld(k + 0), y1 = mp_sld(k + 1), z1 = mp_sld(k + 2);\n"
-        "            const float xv = mp_sld(k + 3), yv = mp_sld(k + 4), zv = mp_sld(k + 5);\n"
-        "            const float rdv = mp_sld(k + 6), crad = mp_sld(k + 7);\n";
-    const char* cyl_load =
-        "            const float* cb = sc.bcyl + o * 4;\n"
-        "            const float ocx = mp_sld(cb + 0), ocy = mp_sld(cb + 1), ocz = mp_sld(cb + 2), orr = mp_sld(cb + 3);\n";
+        "            const float* kp = sc.cap + k * MP_CAP_W;\n"
+        "            const float x1 = mp_sld(kp + 0), y1 = mp_sld(kp + 1), z1 = mp_sld(kp + 2);\n"
+        "            const float xv = mp_sld(kp + 3), yv = mp_sld(kp + 4), zv = mp_sld(kp + 5);\n"
+        "            const float rdv = mp_sld(kp + 6), crad = mp_sld(kp + 7);\n";
     const char* cyl_detail =
-        "            const float* b = sc.cyl + o * MP_CYL_W;\n"
+        "            const float* b = sc.cyl + k * MP_CYL_W;\n"
         "            const float m0 = mp_sld(b + 0), m1 = mp_sld(b + 1), m2 = mp_sld(b + 2), m3 = mp_sld(b + 3);\n"
         "            const float m4 = mp_sld(b + 4), m5 = mp_sld(b + 5), m6 = mp_sld(b + 6), m7 = mp_sld(b + 7);\n"
         "            const float m8 = mp_sld(b + 8), m9 = mp_sld(b + 9), m10 = mp_sld(b + 10), m11 = mp_sld(b + 11);\n"
         "            const float crad = mp_sld(b + 12), hh = mp_sld(b + 13);\n";
+    // the kinds' ranges in the run of bounding spheres
+    const char* ranges =
+        "        const int nb = mp_uniform(sc.nb), ns = mp_uniform(sc.ns), ncap = mp_uniform(sc.ncap), nc = mp_uniform(sc.nc);\n"
+        "        const int e1 = nb + ns, e2 = e1 + ncap, count = e2 + nc;\n";
+    struct Kind {
+        int kind;
+        const char *lo, *hi, *load, *detail;
+    };
     // early-out order: boxes, spheres, capsules, cylinders (cheapest per pair first)
-    // in a team, wave w takes the obstacles o with o % W == w of every kind; the team's early-exit
-    // flag (an LDS read) is looked at every fourth obstacle
-    o << "    template <int MODE>\n    static __device__ __forceinline__ bool env_hit(const float* F, const SceneDev& sc, bool hit, u64 mask, unsigned& work, const Team& T) {\n";
-    o << "        const int o0 = mp_uniform(T.w), os = mp_uniform(T.W);\n" << group_prologue;
-    o << "        for (int o = o0, it = 1; o < mp_uniform(sc.nb); o += os, ++it) {\n" << box_load << env_block(0, false, box_detail)
-      << "            if (mp_stop<MODE>(hit, mask) || ((it & 3) == 0 && T.stopped())) return hit;\n        }\n";
-    o << "        for (int o = o0, it = 1; o < mp_uniform(sc.ns); o += os, ++it) {\n" << sph_load << env_block(1, false, "")
-      << "            if (mp_stop<MODE>(hit, mask) || ((it & 3) == 0 && T.stopped())) return hit;\n        }\n";
-    o << "        for (int o = o0, it = 1; o < mp_uniform(sc.ncap); o += os, ++it) {\n" << cap_load << env_block(2, false, cap_detail)
-      << "            if (mp_stop<MODE>(hit, mask) || ((it & 3) == 0 && T.stopped())) return hit;\n        }\n";
-    o << "        for (int o = o0, it = 1; o < mp_uniform(sc.nc); o += os, ++it) {\n" << cyl_load << env_block(3, false, cyl_detail)
-      << "            if (mp_stop<MODE>(hit, mask) || ((it & 3) == 0 && T.stopped())) return hit;\n        }\n";
-    o << "        return hit;\n    }\n";
-    // full-evaluation costs in the oracle order: spheres, boxes, cylinders, capsules; culled
-    // blocks contribute exact zeros, so skipping them leaves every partial sum unchanged
-    // (per kind into pk[0..3]: the per-constraint costs of the sphere, cuboid, cylinder and
-    // capsule constraints, States.h:205's [constraint][state] rows)
-    o << "    static __device__ __forceinline__ void env_cost(const float* F, const SceneDev& sc, unsigned& work, float* pk) {\n";
-    o << "        float part = 0.0f;\n" << group_prologue;
-    o << "        for (int o = 0; o < mp_uniform(sc.ns); ++o) {\n" << sph_load << env_block(1, true, "") << "        }\n";
-    o << "        pk[0] = part; part = 0.0f;\n";
-    o << "        for (int o = 0; o < mp_uniform(sc.nb); ++o) {\n" << box_load << env_block(0, true, box_detail) << "        }\n";
-    o << "        pk[1] = part; part = 0.0f;\n";
-    o << "        for (int o = 0; o < mp_uniform(sc.nc); ++o) {\n" << cyl_load << env_block(3, true, cyl_detail) << "        }\n";
-    o << "        pk[2] = part; part = 0.0f;\n";
-    o << "        for (int o = 0; o < mp_uniform(sc.ncap); ++o) {\n" << cap_load << env_block(2, true, cap_detail) << "        }\n";
-    o << "        pk[3] = part;\n    }\n";
+    const Kind kinds[4] = {{0, "0", "nb", bound_load, box_detail},
+                           {1, "nb", "e1", sph_load, ""},
+                           {2, "e1", "e2", bound_load, cap_detail},
+                           {3, "e2", "count", bound_load, cyl_detail}};
+    // in a team, wave w takes the near obstacles w, w + W, ... of every kind (all its waves hold the
+    // same states, so they see the same near obstacles); the team's early-exit flag (an LDS read) is
+    // looked at every fourth of them
+    o << "    template <int MODE>\n    static __device__ __forceinline__ bool env_hit(float* F, const SceneDev& sc, mp_f4 ob, bool hit, u64 mask, unsigned& work, const Team& T) {\n";
+    o << "        const int o0 = mp_uniform(T.w), os = mp_uniform(T.W);\n" << ranges << group_prologue;
+    // `seen`: the states the near obstacles are chosen for; a team's waves have to agree on them, so
+    // there it stays as at the start
+    o << "        u64 live = mp_live<MODE>(__ballot(hit), mask);\n        const u64 live0 = live;\n" << group_balls;
+    o << "        for (int base = 0; base < count; base += MP_WAVE) {\n"
+         "            const u64 seen = T.W > 1 ? live0 : live;\n"
+         "            if (base > 0) ob = mp_bound_of_lane(sc, base, count);\n"
+      << group_near << "            work += " << 2 * G * kSph << "u;\n"
+      << "            const u64 near = (" << near_any << ") & mp_bits(base, 0, count);\n";
+    for (const Kind& kd : kinds) {
+        o << "            {\n            u64 m = near & mp_bits(base, " << kd.lo << ", " << kd.hi << ");\n"
+             "            const int nm = __popcll(m);\n"
+             "            m = mp_drop_low(m, o0);\n"
+             "            for (int o = o0, it = 1; o < nm; o += os, ++it) {\n"
+             "            const int l = __builtin_ctzll(m), k = base + l - " << kd.lo << ";\n"
+             "            m = mp_drop_low(m, os);\n"
+          << kd.load << env_block(kd.kind, false, kd.detail)
+          << "            const u64 hb = __ballot(hit);\n"
+             "            if (mp_decides<MODE>(hb, mask) || ((it & 3) == 0 && T.stopped())) return hit;\n"
+             "            live = mp_live<MODE>(hb, mask);\n            }\n            }\n";
+    }
+    o << "        }\n        return hit;\n    }\n";
+    // full-evaluation costs, per kind in index order (the oracle's): spheres, boxes, cylinders,
+    // capsules into pk[0..3], the per-constraint costs of States.h:205's [constraint][state] rows;
+    // culled blocks contribute exact zeros, so skipping them leaves every partial sum unchanged
+    o << "    static __device__ __forceinline__ void env_cost(float* F, const SceneDev& sc, mp_f4 ob, unsigned& work, float* pk) {\n"
+      << ranges << group_prologue << "        const u64 live = ~0ull, seen = live;\n" << group_balls
+      << "        pk[0] = pk[1] = pk[2] = pk[3] = 0.0f;\n"
+         "        for (int base = 0; base < count; base += MP_WAVE) {\n"
+         "            if (base > 0) ob = mp_bound_of_lane(sc, base, count);\n"
+      << group_near << "            work += " << 2 * G * kSph << "u;\n"
+      << "            const u64 near = (" << near_any << ") & mp_bits(base, 0, count);\n";
+    const int row_of[4] = {1, 0, 3, 2};  // box, sphere, capsule, cylinder
+    for (const Kind& kd : kinds) {
+        o << "            {\n            float part = pk[" << row_of[kd.kind] << "];\n"
+             "            for (u64 m = near & mp_bits(base, " << kd.lo << ", " << kd.hi << "); m; m &= m - 1ull) {\n"
+             "            const int l = __builtin_ctzll(m), k = base + l - " << kd.lo << ";\n"
+          << kd.load << env_block(kd.kind, true, kd.detail) << "            }\n            pk[" << row_of[kd.kind] << "] = part;\n            }\n";
+    }
+    o << "        }\n    }\n";
     // joint bounds: BoundaryConstraint.cu:56-92, tolerance 1e-4 on the squared sum
     o << "    static __device__ __forceinline__ float bounds_acc(const float* q) {\n        float acc = 0.0f;\n";
     for (int j = 0; j < m.dof; j++) {
@@ -850,23 +896,23 @@ std::string module_source(const std::vector<const RobotModel*>& robots) {
           << "(const float* q, long long n, float* c) { mp_fk_kernel<" << R << ">(q, n, c); }\n";
         o << "extern \"C\" __global__ void __launch_bounds__(256) mp_poses_" << s
           << "(const float* q, long long n, float* p) { mp_poses_kernel<" << R << ">(q, n, p); }\n";
-        o << "extern \"C\" __global__ void __launch_bounds__(256) mp_check_" << s
-          << "(const float* q, long long n, SceneDev sc, unsigned char* v, float* c, unsigned long long* w) { mp_check_kernel<" << R
-          << ">(q, n, sc, v, c, w); }\n";
-        o << "extern \"C\" __global__ void __launch_bounds__(256) mp_cost_" << s
-          << "(const float* q, long long n, SceneDev sc, float* c, unsigned char* v, float* parts, unsigned long long* w) { mp_cost_kernel<" << R
-          << ">(q, n, sc, c, v, parts, w); }\n";
+        o << "extern \"C\" __global__ void __launch_bounds__(256, 2) mp_check_" << s
+          << "(const float* q, long long n, SceneDev sc, unsigned char* v, float* c, unsigned long long* w, int per_wave) { mp_check_kernel<" << R
+          << ">(q, n, sc, v, c, w, per_wave); }\n";
+        o << "extern \"C\" __global__ void __launch_bounds__(256, 2) mp_cost_" << s
+          << "(const float* q, long long n, SceneDev sc, float* c, unsigned char* v, float* parts, unsigned long long* w, int per_wave) { mp_cost_kernel<" << R
+          << ">(q, n, sc, c, v, parts, w, per_wave); }\n";
         o << "extern \"C\" __global__ void __launch_bounds__(256) mp_sample_" << s
           << "(u64 seed, u64 off, long long n, float* q) { mp_sample_kernel<" << R << ">(seed, off, n, q, MP_SAMPLER_UNIFORM); }\n";
         o << "extern \"C\" __global__ void __launch_bounds__(256) mp_halton_" << s
           << "(u64 seed, u64 off, long long n, float* q) { mp_sample_kernel<" << R << ">(seed, off, n, q, MP_SAMPLER_HALTON); }\n";
-        o << "extern \"C\" __global__ void __launch_bounds__(256) mp_edges_" << s
+        o << "extern \"C\" __global__ void __launch_bounds__(256, 2) mp_edges_" << s
           << "(const float* a, const float* b, int m, float res, SceneDev sc, unsigned char* ok, float* len, unsigned long long* w) { mp_edges_kernel<"
           << R << ">(a, b, m, res, sc, ok, len, w); }\n";
         if (robots.size() == 1) {  // the roadmap planner runs on a single robot's module
             o << "extern \"C\" __global__ void __launch_bounds__(MP_RM_MAX_K) mp_rm_sample_" << s
               << "(RoadmapDev g, SceneDev sc) { mp_rm_sample<" << R << ">(g, sc); }\n";
-            o << "extern \"C\" __global__ void __launch_bounds__(256) mp_rm_edges_" << s
+            o << "extern \"C\" __global__ void __launch_bounds__(256, 2) mp_rm_edges_" << s
               << "(RoadmapDev g, SceneDev sc, unsigned long long* w) { mp_rm_edges<" << R << ">(g, sc, w); }\n";
             o << "extern \"C\" __global__ void __launch_bounds__(64) mp_rm_commit_" << s << "(RoadmapDev g) { mp_rm_commit<"
               << R << "::DOF>(g); }\n";

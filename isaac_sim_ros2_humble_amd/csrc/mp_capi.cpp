@@ -451,6 +451,12 @@ void bound_sphere(float* o, double cx, double cy, double cz, double r) {
 
 void scene_upload(mp_scene* sc, const float* spheres, int ns, const float* boxes, int nb, const float* cyl, int nc,
                   const float* caps, int ncap) {
+    // the bounding spheres of this upload's obstacles in one run: boxes, spheres, capsules, cylinders
+    // (the records keep the places that the capacities gave them)
+    sc->offs[1] = 0;
+    sc->offs[0] = (size_t)4 * nb;
+    sc->offs[5] = sc->offs[0] + (size_t)4 * ns;
+    sc->offs[3] = sc->offs[5] + (size_t)4 * ncap;
     std::vector<float> h(sc->offs[6] + (size_t)MP_CAP_W_H * std::max(sc->cap_k, 1), 0.0f);
     for (int i = 0; i < ns; i++) std::memcpy(&h[sc->offs[0] + 4 * i], spheres + 4 * i, 4 * sizeof(float));
     for (int i = 0; i < nb; i++) {
@@ -510,13 +516,10 @@ int mp_scene_create(const float* spheres, int ns, const float* boxes, int nb, co
         sc->cap_b = nb;
         sc->cap_c = nc;
         sc->cap_k = ncap;
-        sc->offs[0] = 0;
-        sc->offs[1] = sc->offs[0] + (size_t)4 * std::max(ns, 1);
-        sc->offs[2] = sc->offs[1] + (size_t)4 * std::max(nb, 1);
-        sc->offs[3] = sc->offs[2] + (size_t)MP_BOX_W_H * std::max(nb, 1);
-        sc->offs[4] = sc->offs[3] + (size_t)4 * std::max(nc, 1);
-        sc->offs[5] = sc->offs[4] + (size_t)MP_CYL_W_H * std::max(nc, 1);
-        sc->offs[6] = sc->offs[5] + (size_t)4 * std::max(ncap, 1);
+        // [4 floats per obstacle: bounding spheres][box records][cylinder records][capsule records]
+        sc->offs[2] = (size_t)4 * std::max(nb + ns + ncap + nc, 1);
+        sc->offs[4] = sc->offs[2] + (size_t)MP_BOX_W_H * std::max(nb, 1);
+        sc->offs[6] = sc->offs[4] + (size_t)MP_CYL_W_H * std::max(nc, 1);
         size_t total = sc->offs[6] + (size_t)MP_CAP_W_H * std::max(ncap, 1);
         try {
             MP_HIP(hipMalloc(&sc->dev, total * sizeof(float)));
@@ -583,6 +586,19 @@ int mp_scene_destroy(mp_scene* sc) {
 }
 
 // ---------------------------------------------------------------------------------------- kernels
+namespace {
+// States per wave of the check and cost kernels: 64 once the launch fills the chip with them (two
+// waves on each of a CU's four SIMDs, what the kernels' registers allow), else the power of two that
+// still makes that many waves.
+int states_per_wave(int64_t n) {
+    const int64_t waves = (int64_t)std::max(G.num_cus, 1) * 8;
+    int c = 64;
+    while (c > 1 && n <= waves * (c / 2)) c /= 2;
+    return c;
+}
+unsigned state_blocks(int64_t n, int per_wave) { return (unsigned)((n + 4 * per_wave - 1) / (4 * per_wave)); }
+}  // namespace
+
 int mp_fk_spheres(const mp_robot* robot, const float* d_q, int64_t n, float* d_centres, void* stream) {
     return guard([&] {
         need_init();
@@ -613,8 +629,9 @@ int mp_check_states(const mp_robot* robot, const mp_scene* scene, const float* d
         if (n == 0) return;
         long long nn = n;
         mp::SceneDevHost sv = mp::scene_view(scene);
-        void* args[] = {&d_q, &nn, &sv, &d_verdict, &d_centres, &G.work};
-        mp::launch(robot->module->fn("mp_check_0"), (unsigned)((n + 255) / 256), 256, stream_of(stream), args, "check");
+        int per_wave = states_per_wave(n);
+        void* args[] = {&d_q, &nn, &sv, &d_verdict, &d_centres, &G.work, &per_wave};
+        mp::launch(robot->module->fn("mp_check_0"), state_blocks(n, per_wave), 256, stream_of(stream), args, "check");
     });
 }
 
@@ -627,8 +644,9 @@ int mp_state_costs(const mp_robot* robot, const mp_scene* scene, const float* d_
         long long nn = n;
         mp::SceneDevHost sv = mp::scene_view(scene);
         float* d_parts = nullptr;
-        void* args[] = {&d_q, &nn, &sv, &d_cost, &d_verdict, &d_parts, &G.work};
-        mp::launch(robot->module->fn("mp_cost_0"), (unsigned)((n + 255) / 256), 256, stream_of(stream), args, "cost");
+        int per_wave = states_per_wave(n);
+        void* args[] = {&d_q, &nn, &sv, &d_cost, &d_verdict, &d_parts, &G.work, &per_wave};
+        mp::launch(robot->module->fn("mp_cost_0"), state_blocks(n, per_wave), 256, stream_of(stream), args, "cost");
     });
 }
 
@@ -640,8 +658,9 @@ int mp_constraint_costs(const mp_robot* robot, const mp_scene* scene, const floa
         if (n == 0) return;
         long long nn = n;
         mp::SceneDevHost sv = mp::scene_view(scene);
-        void* args[] = {&d_q, &nn, &sv, &d_cost, &d_verdict, &d_parts, &G.work};
-        mp::launch(robot->module->fn("mp_cost_0"), (unsigned)((n + 255) / 256), 256, stream_of(stream), args, "cost");
+        int per_wave = states_per_wave(n);
+        void* args[] = {&d_q, &nn, &sv, &d_cost, &d_verdict, &d_parts, &G.work, &per_wave};
+        mp::launch(robot->module->fn("mp_cost_0"), state_blocks(n, per_wave), 256, stream_of(stream), args, "cost");
     });
 }
 

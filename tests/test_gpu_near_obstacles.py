@@ -1,0 +1,78 @@
+"""The check kernels' choice of near obstacles: scenes whose obstacle count sits at the edges of the
+64-obstacle chunks, batches at the edges of the states-per-wave split, a NaN state among free ones,
+and a scene that shrinks.  Verdicts, costs and motions equal the oracle's bit for bit (the cull only
+skips what cannot touch, so there is no tolerance)."""
+import numpy as np
+import pytest
+
+import oracle
+from isaac_sim_ros2_humble_amd import native, workloads
+from isaac_sim_ros2_humble_amd.scene import Scene, capsule_record, random_rotation
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def robots(fr3, fetch):
+    native.init(0)
+    return {"fr3": native.Robot(fr3), "fetch": native.Robot(fetch)}
+
+
+def _scene(model, count, seed):
+    """`count` obstacles of all four kinds, every fourth a capsule."""
+    rng = np.random.default_rng(seed)
+    lo, hi, keep = workloads.workspace(model)
+    ncap = count // 4
+    s = workloads.random_scene(rng, count - ncap, lo, hi, keep)
+    caps = [capsule_record(rng.uniform([0.4, 0.4, 0.1], [1.0, 1.0, 1.4]), random_rotation(rng), rng.uniform(0.02, 0.08),
+                           rng.uniform(0.1, 0.5)) for _ in range(ncap)]
+    s.capsules = np.array(caps, np.float32).reshape(-1, 7)
+    assert s.num_obstacles == count
+    return s
+
+
+@pytest.mark.parametrize("name,count,n", [
+    ("fr3", 1, 1), ("fr3", 63, 65), ("fr3", 64, 2048), ("fr3", 65, 2049), ("fetch", 127, 300), ("fetch", 129, 4097),
+    ("fr3", 200, 131073)])
+def test_checks_at_chunk_edges(name, count, n, robots, request):
+    m = request.getfixturevalue(name)
+    orc = request.getfixturevalue("orc_" + name)
+    scene = _scene(m, count, seed=count)
+    q = workloads.uniform_configs(m, n, np.random.default_rng(n))
+    ns, osc = native.Scene(scene), oracle.OracleScene(scene)
+    v = native.check_states(robots[name], ns, q)
+    vo, co, _, _ = oracle.check(orc, osc, q, want_cost=True, nthreads=8)
+    assert np.array_equal(v, vo)
+    cost, vc = native.state_costs(robots[name], ns, q)
+    assert np.array_equal(cost, co) and np.array_equal(vc, vo)
+    k = min(n // 2, 200)
+    if k:
+        ok, ln = native.check_edges(robots[name], ns, q[:k], q[k:2 * k], 0.02)
+        oko, lno = oracle.edges(orc, osc, q[:k], q[k:2 * k], 0.02)
+        assert np.array_equal(ok, oko) and np.array_equal(ln, lno)
+
+
+def test_nan_state_does_not_hide_obstacles(fr3, orc_fr3, robots):
+    # the lanes that the waves' balls are centred on (16, 48) hold NaN or infinite states
+    scene = _scene(fr3, 64, seed=3)
+    q = workloads.uniform_configs(fr3, 1 << 18, np.random.default_rng(4))
+    q[16::64] = np.nan
+    q[48::128, 3] = np.inf
+    keep = np.isfinite(q).all(axis=1)
+    v = native.check_states(robots["fr3"], native.Scene(scene), q)
+    vo, _, _, _ = oracle.check(orc_fr3, oracle.OracleScene(scene), q[keep], nthreads=8)
+    assert np.array_equal(v[keep], vo)
+
+
+def test_scene_update_to_fewer_obstacles(fr3, orc_fr3, robots):
+    big, small = _scene(fr3, 130, seed=5), _scene(fr3, 37, seed=6)
+    ns = native.Scene(big)
+    q = workloads.uniform_configs(fr3, 3000, np.random.default_rng(7))
+    for s in (big, small, big):
+        keep = Scene(spheres=s.spheres[:len(big.spheres)], boxes=s.boxes[:len(big.boxes)],
+                     cylinders=s.cylinders[:len(big.cylinders)], capsules=s.capsules[:len(big.capsules)])
+        ns.update(keep)
+        vo, co, _, _ = oracle.check(orc_fr3, oracle.OracleScene(keep), q, want_cost=True, nthreads=8)
+        cost, v = native.state_costs(robots["fr3"], ns, q)
+        assert np.array_equal(v, vo) and np.array_equal(cost, co)
+        assert np.array_equal(native.check_states(robots["fr3"], ns, q), vo)
