@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstdio>
 #include <array>
+#include <functional>
 #include <map>
 #include <sstream>
 
@@ -270,16 +271,22 @@ std::vector<SphereLink> sphere_links(const RobotModel& m) {
 // flop costs of the planning cost model (FMA = 2, add/mul/min/max/cmp = 1)
 constexpr int kXform = 18, kSelf = 9, kSph = 11, kBox = 34, kCyl = 35, kCap = 28;
 constexpr int kCentreChunk = 16;  // spheres per staged chunk; the LDS row is MP_CENTRE_ROW floats
+constexpr int kPoseChunk = 2;     // links per staged chunk (128 bytes per state); the LDS row is MP_POSE_ROW floats
+// LDS of the FK kernel's tile: whole rows of centres for as many states of a wave as fit.  40 KB keep
+// four one-wave workgroups on a CU, enough to cover the stores' latency with the next states' FK.
+constexpr int kCentreTileFloats = 12 * 1024;
 
 }  // namespace
 
 // Link frames of every link (KernelGenerator.h:254-348 composition order), emitted into E with
-// constant folding; returns the symbolic frames.
-std::vector<Aff> emit_frames(Emitter& E, const RobotModel& m, int& fk_flops) {
+// constant folding; returns the symbolic frames.  `done` (optional) is called after each link's frame.
+std::vector<Aff> emit_frames(Emitter& E, const RobotModel& m, int& fk_flops,
+                             const std::function<void(int, const Aff&)>& done = nullptr) {
     std::vector<Aff> T(m.L);
     T[0] = identity();
     int ntrig = 0;
     for (int i = 1; i < m.L; i++) {
+        if (done) done(i - 1, T[i - 1]);
         const Aff& P = T[m.parent[i]];
         Aff O;
         for (int a = 0; a < 3; a++) {
@@ -323,6 +330,7 @@ std::vector<Aff> emit_frames(Emitter& E, const RobotModel& m, int& fk_flops) {
             T[i] = P;
         }
     }
+    if (done) done(m.L - 1, T[m.L - 1]);
     return T;
 }
 
@@ -331,22 +339,27 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     Emitter E;
     int fk_flops = 0;
     const std::vector<Aff> T = emit_frames(E, m, fk_flops);
-    // link poses [L][16], row-major 4x4 with the last row (0, 0, 0, 1)
+    // link poses [L][16], row-major 4x4 with the last row (0, 0, 0, 1), staged through LDS in chunks
+    // of kPoseChunk links: a wave's poses are 64 L apart per state, so a lane's own 16-byte stores
+    // would touch 64 lines each; from the tile, consecutive lanes write a state's whole chunk
     std::string poses_body;
     {
         Emitter EP;
         int unused = 0;
-        const std::vector<Aff> TP = emit_frames(EP, m, unused);
-        for (int i = 0; i < m.L; i++) {
+        emit_frames(EP, m, unused, [&](int i, const Aff& F) {
+            const int c = i % kPoseChunk, first = i - c, links = std::min(kPoseChunk, m.L - first);
             for (int a = 0; a < 3; a++) {
                 for (int b = 0; b < 3; b++)
-                    EP.os << EP.ind << "P[" << 16 * i + 4 * a + b << "] = " << EP.ref(TP[i].R[3 * a + b]) << ";\n";
-                EP.os << EP.ind << "P[" << 16 * i + 4 * a + 3 << "] = " << EP.ref(TP[i].t[a]) << ";\n";
+                    EP.os << EP.ind << "P[" << 16 * c + 4 * a + b << "] = " << EP.ref(F.R[3 * a + b]) << ";\n";
+                EP.os << EP.ind << "P[" << 16 * c + 4 * a + 3 << "] = " << EP.ref(F.t[a]) << ";\n";
             }
-            EP.os << EP.ind << "P[" << 16 * i + 12 << "] = 0.0f; P[" << 16 * i + 13 << "] = 0.0f; P[" << 16 * i + 14
-                  << "] = 0.0f; P[" << 16 * i + 15 << "] = 1.0f;\n";
-        }
-        poses_body = EP.os.str();
+            EP.os << EP.ind << "P[" << 16 * c + 12 << "] = 0.0f; P[" << 16 * c + 13 << "] = 0.0f; P[" << 16 * c + 14
+                  << "] = 0.0f; P[" << 16 * c + 15 << "] = 1.0f;\n";
+            if (c == links - 1)
+                EP.os << EP.ind << "mp_copy_rows<" << 4 * links << ", MP_POSE_ROW, " << 16 * m.L << ">(tile, out + " << 16 * first
+                      << ", live);\n";
+        });
+        poses_body = "        float* P = tile + (threadIdx.x & (MP_WAVE - 1)) * MP_POSE_ROW;\n" + EP.os.str();
     }
     const std::vector<SphereLink> SL = sphere_links(m);
     const int NL = (int)SL.size();
@@ -743,8 +756,12 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     o << "    static constexpr unsigned FK_WORK = " << fk_flops << "u;\n";
     o << "    static __device__ __forceinline__ void fk(const float* q, float* F) {\n" << fk_body << "    }\n";
     o << "    static constexpr int NLINK = " << m.L << ";\n";
-    o << "    static __device__ __forceinline__ void poses(const float* q, float* P) {\n" << poses_body << "    }\n";
+    o << "    static __device__ __forceinline__ void poses(const float* q, float* out, int live, float* tile) {\n" << poses_body << "    }\n";
     o << "    static __device__ __forceinline__ void write_centres(const float* F, float* out) {\n" << centres_body << "    }\n";
+    // states of a wave whose centres fit the FK kernel's tile at once (a power of two)
+    int crows = 64;
+    while (crows > 4 && crows * 3 * m.S > kCentreTileFloats) crows /= 2;
+    o << "    static constexpr int CROWS = " << crows << ";\n";
     o << "    // out: the wave's first configuration; live: its configurations below n; tile: the wave's\n"
          "    // LDS tile of MP_WAVE x MP_CENTRE_ROW floats\n"
          "    static __device__ __forceinline__ void write_centres_staged(const float* F, float* out, int live, float* tile) {\n"
@@ -892,7 +909,7 @@ std::string module_source(const std::vector<const RobotModel*>& robots) {
     o << kernel_template_body();
     for (size_t k = 0; k < robots.size(); k++) {
         std::string R = "Robot" + std::to_string(k), s = std::to_string(k);
-        o << "extern \"C\" __global__ void __launch_bounds__(256) mp_fk_" << s
+        o << "extern \"C\" __global__ void __launch_bounds__(64) mp_fk_" << s
           << "(const float* q, long long n, float* c) { mp_fk_kernel<" << R << ">(q, n, c); }\n";
         o << "extern \"C\" __global__ void __launch_bounds__(256) mp_poses_" << s
           << "(const float* q, long long n, float* p) { mp_poses_kernel<" << R << ">(q, n, p); }\n";

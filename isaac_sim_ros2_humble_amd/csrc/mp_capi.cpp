@@ -606,7 +606,7 @@ int mp_fk_spheres(const mp_robot* robot, const float* d_q, int64_t n, float* d_c
         if (n == 0) return;
         long long nn = n;
         void* args[] = {&d_q, &nn, &d_centres};
-        mp::launch(robot->module->fn("mp_fk_0"), (unsigned)((n + 255) / 256), 256, stream_of(stream), args, "fk");
+        mp::launch(robot->module->fn("mp_fk_0"), (unsigned)((n + 63) / 64), 64, stream_of(stream), args, "fk");
     });
 }
 
@@ -687,7 +687,10 @@ int mp_nn_argmin(const float* d_tree, int n_nodes, int capacity, int dof, const 
         if (nq == 0) return;
         auto mod = mp::get_module({});
         void* args[] = {&d_tree, &n_nodes, &capacity, &dof, &d_q, &nq, &d_idx};
-        mp::launch(mod->fn("mp_nn_generic"), (unsigned)((nq + 3) / 4), 256, stream_of(stream), args, "nn");
+        // two queries per workgroup (the kernel's MP_NN_Q), up to 16 waves (its launch bound) that share
+        // the nodes: one wave per 256 nodes, below which more waves cost more than they save
+        const int waves = std::min(16, std::max(1, (n_nodes + 255) / 256));
+        mp::launch(mod->fn("mp_nn_generic"), (unsigned)((nq + 1) / 2), 64u * waves, stream_of(stream), args, "nn");
     });
 }
 
