@@ -364,22 +364,19 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     const std::vector<SphereLink> SL = sphere_links(m);
     const int NL = (int)SL.size();
     fk_flops += kXform * NL;
-    // F layout per sphere link k: [k*15 + 0..8] rotation (row major), [+9..11] translation,
-    // [+12..14] world bounding-sphere centre.  Constant entries are returned as constants.
-    std::vector<std::vector<V>> FV(NL, std::vector<V>(15));
+    // F layout per sphere link k: [k*12 + 0..8] rotation (row major), [+9..11] translation.  Constant
+    // entries are returned as constants.  A link's bounding-sphere centre is computed where it is used
+    // (link_centre): held as well, the centres of Fetch's 14 links take 42 registers that the near
+    // obstacles' tests need.
+    std::vector<std::vector<V>> FV(NL, std::vector<V>(12));
     for (int k = 0; k < NL; k++) {
         const Aff& M = T[SL[k].link];
-        V b[3];
-        for (int a = 0; a < 3; a++)
-            b[a] = E.row(M.R[3 * a], K((float)SL[k].c[0]), M.R[3 * a + 1], K((float)SL[k].c[1]), M.R[3 * a + 2],
-                         K((float)SL[k].c[2]), M.t[a]);
         for (int e = 0; e < 9; e++) FV[k][e] = M.R[e];
         for (int a = 0; a < 3; a++) FV[k][9 + a] = M.t[a];
-        for (int a = 0; a < 3; a++) FV[k][12 + a] = b[a];
-        for (int e = 0; e < 15; e++) {
+        for (int e = 0; e < 12; e++) {
             if (!FV[k][e].k) {
-                E.os << E.ind << "F[" << k * 15 + e << "] = " << FV[k][e].e << ";\n";
-                FV[k][e] = V{false, 0.0f, "F[" + std::to_string(k * 15 + e) + "]"};
+                E.os << E.ind << "F[" << k * 12 + e << "] = " << FV[k][e].e << ";\n";
+                FV[k][e] = V{false, 0.0f, "F[" + std::to_string(k * 12 + e) + "]"};
             }
         }
     }
@@ -393,6 +390,11 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     auto centre = [&](Emitter& X, int s, V out[3]) {
         const std::vector<V>& f = FV[slk[s]];
         V p[3] = {K(m.sphere_pos[3 * s]), K(m.sphere_pos[3 * s + 1]), K(m.sphere_pos[3 * s + 2])};
+        for (int a = 0; a < 3; a++) out[a] = X.row(f[3 * a], p[0], f[3 * a + 1], p[1], f[3 * a + 2], p[2], f[9 + a]);
+    };
+    auto link_centre = [&](Emitter& X, int k, V out[3]) {
+        const std::vector<V>& f = FV[k];
+        V p[3] = {K((float)SL[k].c[0]), K((float)SL[k].c[1]), K((float)SL[k].c[2])};
         for (int a = 0; a < 3; a++) out[a] = X.row(f[3 * a], p[0], f[3 * a + 1], p[1], f[3 * a + 2], p[2], f[9 + a]);
     };
     auto named = [&](Emitter& X, const V& v) -> std::string { return X.ref(v); };
@@ -463,7 +465,19 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     auto self_body = [&](bool cost) {
         Emitter X;
         int blk = 0;
-        for (const LP& lp : lps) {
+        // verdicts: the link pairs with the most sphere pairs last, where their held centres find the
+        // registers of the frames and link centres that no later pair needs; a team's waves also get
+        // alternate ones.  Costs add up in the oracle's order.
+        std::vector<LP> order = lps;
+        if (!cost)
+            std::stable_sort(order.begin(), order.end(), [](const LP& a, const LP& b) { return a.pairs.size() < b.pairs.size(); });
+        std::vector<std::array<V, 3>> B0(NL);
+        for (int k = 0; k < NL; k++) {
+            V b[3];
+            link_centre(X, k, b);
+            B0[k] = {b[0], b[1], b[2]};
+        }
+        for (const LP& lp : order) {
             const SphereLink& A = SL[lp.a];
             const SphereLink& B = SL[lp.b];
             float cull = (float)((A.R + B.R + kCullMargin) * (A.R + B.R + kCullMargin));
@@ -472,7 +486,7 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
             blk++;
             X.os << "        {\n";
             V d[3];
-            for (int a = 0; a < 3; a++) d[a] = X.sub(FV[lp.a][12 + a], FV[lp.b][12 + a]);
+            for (int a = 0; a < 3; a++) d[a] = X.sub(B0[lp.a][a], B0[lp.b][a]);
             V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
             X.os << "        work += " << kSelf << "u;\n";
             X.os << "        if (__ballot(" << X.ref(d2) << " < " << lit(cull) << ")" << (cost ? "" : " & live") << ") {\n";
@@ -487,9 +501,20 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                 const SphereLink& Sk = a_small ? B : A;
                 std::map<int, std::array<V, 3>> held;
                 for (int s : Hk.spheres) { V c[3]; centre(X, s, c); held[s] = {c[0], c[1], c[2]}; }
+                // a streamed sphere's pairs are skipped when no live lane's sphere reaches the held
+                // link's bounding sphere (from three pairs on, which cost more than the test)
+                const bool cull_sphere = Hk.spheres.size() >= 3;
+                const int kh = a_small ? lp.a : lp.b;
                 for (int s : Sk.spheres) {
                     V c[3];
                     centre(X, s, c);
+                    if (cull_sphere) {
+                        V e[3];
+                        for (int a = 0; a < 3; a++) e[a] = X.sub(c[a], B0[kh][a]);
+                        V dd = X.dot3(e[0], e[0], e[1], e[1], e[2], e[2]);
+                        const double reach = Hk.R + m.sphere_r[s] + kCullMargin;
+                        X.os << "            if (__ballot(" << X.ref(dd) << " < " << lit((float)(reach * reach)) << ") & live) {\n";
+                    }
                     for (int hsph : Hk.spheres) {
                         float thr, sr;
                         pair_thr(std::min(hsph, s), std::max(hsph, s), thr, sr);
@@ -501,6 +526,7 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                         V dd = X.dot3(e[0], e[0], e[1], e[1], e[2], e[2]);
                         X.os << "            h |= " << X.ref(dd) << " < " << lit(std::min(thr, sqrt_threshold(sr))) << ";\n";
                     }
+                    if (cull_sphere) X.os << "            }\n";
                 }
                 X.os << "            const u64 hb = __ballot(h);\n"
                         "            if (mp_decides<MODE>(hb, mask)) return h;\n"
@@ -537,72 +563,34 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
         return X.os.str();
     };
 
-    // ---------------------------------------------------------------- link groups
-    // Obstacle-level culling: the sphere links are split into contiguous groups; per lane, a
-    // group's bounding sphere is centred on its middle link's bounding-sphere centre with radius
-    // max(|b_k - c| + R_k) + 2 margins.  An obstacle whose bounding sphere misses every lane's
-    // group sphere cannot reach any link of the group (triangle inequality), so the group's link
-    // tests are skipped.
-    std::vector<std::vector<int>> groups;
-    {
-        const int G = NL <= 2 ? 1 : std::min(4, (NL + 2) / 3);
-        for (int g = 0; g < G; g++) {
-            std::vector<int> v;
-            for (int k = g * NL / G; k < (g + 1) * NL / G; k++) v.push_back(k);
-            if (!v.empty()) groups.push_back(v);
-        }
+    // ---------------------------------------------------------------- near obstacles
+    // Which of the wave's obstacles of a chunk each sphere-carrying link may reach (bit l: lane l's):
+    // the link's balls over the wave's states against one obstacle per lane (mp_half_balls, mp_near).
+    // Each chunk computes the balls anew: kept from the first chunk in lanes, they cost as much to
+    // put there and read back.  A link that nothing moves has the same centre in every lane.
+    std::string link_near = "            const float reach = mp_bound_reach(ob);\n", near_any = NL == 0 ? "0ull" : "";
+    for (int k = 0; k < NL; k++) {
+        const std::string n = std::to_string(k);
+        Emitter X;
+        X.pfx = "b" + n + "_";
+        X.ind = "            ";
+        V b[3];
+        link_centre(X, k, b);
+        const std::string r = "reach + " + lit((float)(SL[k].R + 2.0 * kCullMargin));
+        const std::string at = X.ref(b[0]) + ", " + X.ref(b[1]) + ", " + X.ref(b[2]);
+        if (b[0].k && b[1].k && b[2].k)
+            link_near += "            const u64 lm" + n + " = mp_near_fixed(ob, " + r + ", " + at + ");\n";
+        else
+            link_near += X.os.str() + "            const u64 lm" + n + " = mp_near(ob, " + r + ", mp_half_balls(" + at + ", live), live);\n";
+        near_any += (k ? " | lm" : "lm") + n;
     }
-    Emitter GP;
-    GP.pfx = "gp";
-    std::vector<std::array<V, 4>> gsph;
-    for (const auto& g : groups) {
-        const int km = g[g.size() / 2];
-        V c[3] = {FV[km][12], FV[km][13], FV[km][14]};
-        V r = K(0.0f);
-        bool first = true;
-        for (int k : g) {
-            const float Rk = (float)(SL[k].R + 2.0 * kCullMargin);
-            V term;
-            if (k == km) {
-                term = K(Rk);
-            } else {
-                V d[3] = {GP.sub(FV[k][12], c[0]), GP.sub(FV[k][13], c[1]), GP.sub(FV[k][14], c[2])};
-                V dd = GP.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
-                // a cull's radius: the hardware square root, rounded up by 1e-6 relative
-                term = dd.k ? K(std::sqrt(dd.c) * 1.000001f + Rk)
-                            : GP.tmp("__builtin_fmaf(__builtin_amdgcn_sqrtf(" + GP.ref(dd) + "), 1.000001f, " + lit(Rk) + ")");
-            }
-            if (first) {
-                r = term;
-                first = false;
-            } else if (r.k && term.k) {
-                r = K(std::max(r.c, term.c));
-            } else {
-                r = GP.tmp("fmaxf(" + GP.ref(r) + ", " + GP.ref(term) + ")");
-            }
-        }
-        gsph.push_back({c[0], c[1], c[2], r});
-    }
-    const std::string group_prologue = GP.os.str();
-    const int G = (int)groups.size();
-    // the groups' balls over the wave's live states (mp_half_balls), and the near obstacles of the
-    // chunk of 64 from `base` on
-    std::string group_balls, group_near = "            const float reach = mp_bound_reach(ob);\n", near_any;
-    for (int gi = 0; gi < G; gi++) {
-        const std::string g = std::to_string(gi);
-        group_balls += "        const HalfBalls hb" + g + " = mp_half_balls(" + GP.ref(gsph[gi][0]) + ", " + GP.ref(gsph[gi][1]) +
-                       ", " + GP.ref(gsph[gi][2]) + ", " + GP.ref(gsph[gi][3]) + ", live);\n";
-        group_near += "            const u64 gm" + g + " = mp_near(ob, reach, hb" + g + ", seen);\n";
-        near_any += (gi ? " | gm" : "gm") + g;
-    }
-    if (G == 0) near_any = "0ull";
     // The link frames made opaque at the head of each near obstacle's block: otherwise the sphere
     // centres, which do not change from obstacle to obstacle, are moved out of the loop, far more of
     // them than there are registers (FR3's check kernel 258 -> 212 VGPRs, two waves per SIMD again;
     // mp_plan 383 -> 308)
     std::string pin;
     for (int k = 0; k < NL; k++)
-        for (int e = 0; e < 15; e++)
+        for (int e = 0; e < 12; e++)
             if (!FV[k][e].k) pin += "            asm volatile(\"\" : \"+v\"(" + FV[k][e].e + "));\n";
 
     // ---------------------------------------------------------------- environment blocks
@@ -613,27 +601,14 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
         Emitter X;
         V mm[12];
         for (int i = 0; i < 12; i++) mm[i] = V{false, 0.0f, "m" + std::to_string(i)};
-        // obstacle bounding sphere (centre, radius): the sphere itself, or the record's bound
-        const V oc[3] = {V{false, 0.0f, kind == 1 ? "ox" : "ocx"}, V{false, 0.0f, kind == 1 ? "oy" : "ocy"},
-                         V{false, 0.0f, kind == 1 ? "oz" : "ocz"}};
-        const std::string orr = kind == 1 ? "orad" : "orr";
         X.os << pin << detail;
-        for (int gi = 0; gi < G; gi++) {
-        // the groups whose ball the obstacle reaches, then those with a live state near it
-        X.os << "            if ((gm" << gi << " >> l) & 1ull) {\n";
-        {
-            V gd[3] = {X.sub(gsph[gi][0], oc[0]), X.sub(gsph[gi][1], oc[1]), X.sub(gsph[gi][2], oc[2])};
-            V gd2 = X.dot3(gd[0], gd[0], gd[1], gd[1], gd[2], gd[2]);
-            V gs = X.tmp(X.ref(gsph[gi][3]) + " + " + orr);
-            X.os << "            work += " << kSph << "u;\n";
-            X.os << "            if (__ballot(" << X.ref(gd2) << " < " << X.ref(gs) << " * " << X.ref(gs) << ") & live) {\n";
-        }
-        for (int k : groups[gi]) {
+        for (int k = 0; k < NL; k++) {
             const SphereLink& L = SL[k];
             float Rm = (float)(L.R + kCullMargin);
             int n = (int)L.spheres.size();
-            X.os << "            {\n";
-            V b[3] = {FV[k][12], FV[k][13], FV[k][14]};
+            X.os << "            if ((lm" << k << " >> l) & 1ull) {\n";
+            V b[3];
+            link_centre(X, k, b);
             std::string cond;
             int tcost = kind == 0 ? kBox : kind == 1 ? kSph : kind == 2 ? kCap : kCyl;
             if (kind == 0 || kind == 3) {
@@ -661,7 +636,7 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
                 cond = X.ref(d2) + " < " + X.ref(sr) + " * " + X.ref(sr);
             }
             X.os << "            work += " << tcost << "u;\n";
-            X.os << "            if (__ballot(" << cond << ") & live) {\n";
+            X.os << "            if (__ballot(" << cond << ")" << (cost ? "" : " & live") << ") {\n";
             X.os << "                work += " << n * (kXform + tcost) << "u;\n";
             // spheres and capsules: contact <=> d2 < (r+R)^2 and sqrtf(d2) < r+R (the cost
             // (r+R) - sqrtf(d2) is then > 0); a fast test with a 1e-6 relative margin, then the
@@ -740,8 +715,6 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
             }
             X.os << "            }\n            }\n";
         }
-        X.os << "            }\n            }\n";
-        }
         return X.os.str();
     };
 
@@ -752,7 +725,7 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     o << "    static constexpr int S = " << m.S << ";\n";
     o << "    static constexpr int P = " << P << ";\n";
     o << "    static constexpr int NL = " << NL << ";\n";
-    o << "    static constexpr int NF = " << NL * 15 << ";\n";
+    o << "    static constexpr int NF = " << NL * 12 << ";\n";
     o << "    static constexpr unsigned FK_WORK = " << fk_flops << "u;\n";
     o << "    static __device__ __forceinline__ void fk(const float* q, float* F) {\n" << fk_body << "    }\n";
     o << "    static constexpr int NLINK = " << m.L << ";\n";
@@ -773,63 +746,57 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
       << self_body(false) << "        return h;\n    }\n";
     o << "    static __device__ __forceinline__ float self_cost(const float* F, unsigned& work) {\n        float part = 0.0f;\n"
       << self_body(true) << "        return part;\n    }\n";
-    // a near obstacle's bounding sphere comes from the lane that tested it, its record by scalar loads
-    const char* bound_load =
-        "            const float ocx = mp_lane(ob.x, l), ocy = mp_lane(ob.y, l), ocz = mp_lane(ob.z, l), orr = mp_lane(ob.w, l);\n";
+    // a sphere obstacle is its bounding sphere, which a lane holds; the others' records come by scalar loads
     const char* sph_load =
         "            const float ox = mp_lane(ob.x, l), oy = mp_lane(ob.y, l), oz = mp_lane(ob.z, l), orad = mp_lane(ob.w, l);\n";
-    const char* box_detail =
-        "            const float* b = sc.box + k * MP_BOX_W;\n"
-        "            const float m0 = mp_sld(b + 0), m1 = mp_sld(b + 1), m2 = mp_sld(b + 2), m3 = mp_sld(b + 3);\n"
-        "            const float m4 = mp_sld(b + 4), m5 = mp_sld(b + 5), m6 = mp_sld(b + 6), m7 = mp_sld(b + 7);\n"
-        "            const float m8 = mp_sld(b + 8), m9 = mp_sld(b + 9), m10 = mp_sld(b + 10), m11 = mp_sld(b + 11);\n"
-        "            const float lox = mp_sld(b + 12), loy = mp_sld(b + 13), loz = mp_sld(b + 14);\n"
-        "            const float hix = mp_sld(b + 15), hiy = mp_sld(b + 16), hiz = mp_sld(b + 17);\n";
-    const char* cap_detail =
-        "            const float* kp = sc.cap + k * MP_CAP_W;\n"
-        "            const float x1 = mp_sld(kp + 0), y1 = mp_sld(kp + 1), z1 = mp_sld(kp + 2);\n"
-        "            const float xv = mp_sld(kp + 3), yv = mp_sld(kp + 4), zv = mp_sld(kp + 5);\n"
-        "            const float rdv = mp_sld(kp + 6), crad = mp_sld(kp + 7);\n";
-    const char* cyl_detail =
-        "            const float* b = sc.cyl + k * MP_CYL_W;\n"
-        "            const float m0 = mp_sld(b + 0), m1 = mp_sld(b + 1), m2 = mp_sld(b + 2), m3 = mp_sld(b + 3);\n"
-        "            const float m4 = mp_sld(b + 4), m5 = mp_sld(b + 5), m6 = mp_sld(b + 6), m7 = mp_sld(b + 7);\n"
-        "            const float m8 = mp_sld(b + 8), m9 = mp_sld(b + 9), m10 = mp_sld(b + 10), m11 = mp_sld(b + 11);\n"
-        "            const float crad = mp_sld(b + 12), hh = mp_sld(b + 13);\n";
+    auto fields = [](const std::vector<std::string>& names) {
+        std::string t;
+        for (size_t f = 0; f < names.size(); f++)
+            t += "            const float " + names[f] + " = mp_sld(rec + " + std::to_string(f) + ");\n";
+        return t;
+    };
+    const std::vector<std::string> pose = {"m0", "m1", "m2", "m3", "m4", "m5", "m6", "m7", "m8", "m9", "m10", "m11"};
+    std::vector<std::string> box_names = pose, cyl_names = pose;
+    for (const char* f : {"lox", "loy", "loz", "hix", "hiy", "hiz"}) box_names.push_back(f);
+    for (const char* f : {"crad", "hh"}) cyl_names.push_back(f);
+    const std::string box_detail = fields(box_names), cyl_detail = fields(cyl_names),
+                      cap_detail = fields({"x1", "y1", "z1", "xv", "yv", "zv", "rdv", "crad"});
     // the kinds' ranges in the run of bounding spheres
     const char* ranges =
         "        const int nb = mp_uniform(sc.nb), ns = mp_uniform(sc.ns), ncap = mp_uniform(sc.ncap), nc = mp_uniform(sc.nc);\n"
         "        const int e1 = nb + ns, e2 = e1 + ncap, count = e2 + nc;\n";
     struct Kind {
         int kind;
-        const char *lo, *hi, *load, *detail;
+        const char *lo, *hi, *record;  // record: of the obstacle in lane l (scalar loads), if it has one
+        std::string load, detail;
     };
-    // early-out order: boxes, spheres, capsules, cylinders (cheapest per pair first)
-    const Kind kinds[4] = {{0, "0", "nb", bound_load, box_detail},
-                           {1, "nb", "e1", sph_load, ""},
-                           {2, "e1", "e2", bound_load, cap_detail},
-                           {3, "e2", "count", bound_load, cyl_detail}};
-    // in a team, wave w takes the near obstacles w, w + W, ... of every kind (all its waves hold the
-    // same states, so they see the same near obstacles); the team's early-exit flag (an LDS read) is
-    // looked at every fourth of them
+    // order of the tests: spheres (the cheapest, and they need no record), boxes, capsules, cylinders
+    const Kind kinds[4] = {{1, "nb", "e1", "", sph_load, ""},
+                           {0, "0", "nb", "sc.box + (base + l * os + o0) * MP_BOX_W", "", box_detail},
+                           {2, "e1", "e2", "sc.cap + (base + l * os + o0 - e1) * MP_CAP_W", "", cap_detail},
+                           {3, "e2", "count", "sc.cyl + (base + l * os + o0 - e2) * MP_CYL_W", "", cyl_detail}};
+    auto near_of = [](const Kind& kd) {
+        return "            {\n            u64 m = near & mp_lanes_of(base, " + std::string(kd.lo) + ", " + kd.hi + ", T);\n";
+    };
+    auto step = [](const Kind& kd) {
+        return "            const int l = __builtin_ctzll(m);\n            m &= m - 1ull;\n" +
+               (*kd.record ? "            const float* rec = " + std::string(kd.record) + ";\n" : std::string());
+    };
+    // The near obstacles of a kind that the wave takes: its lanes' bits, number o of the team's (o % W
+    // == w).  The team's early-exit flag (an LDS read) is looked at every fourth of them.
     o << "    template <int MODE>\n    static __device__ __forceinline__ bool env_hit(float* F, const SceneDev& sc, mp_f4 ob, bool hit, u64 mask, unsigned& work, const Team& T) {\n";
-    o << "        const int o0 = mp_uniform(T.w), os = mp_uniform(T.W);\n" << ranges << group_prologue;
-    // `seen`: the states the near obstacles are chosen for; a team's waves have to agree on them, so
-    // there it stays as at the start
-    o << "        u64 live = mp_live<MODE>(__ballot(hit), mask);\n        const u64 live0 = live;\n" << group_balls;
-    o << "        for (int base = 0; base < count; base += MP_WAVE) {\n"
-         "            const u64 seen = T.W > 1 ? live0 : live;\n"
-         "            if (base > 0) ob = mp_bound_of_lane(sc, base, count);\n"
-      << group_near << "            work += " << 2 * G * kSph << "u;\n"
-      << "            const u64 near = (" << near_any << ") & mp_bits(base, 0, count);\n";
+    o << "        const int o0 = mp_uniform(T.w), os = mp_uniform(T.W);\n" << ranges;
+    o << "        u64 live = mp_live<MODE>(__ballot(hit), mask);\n"
+         "        const int chunk = MP_WAVE * os;\n";
+    o << "        for (int base = 0; base < count; base += chunk) {\n"
+         "            if (base > 0) ob = mp_bound_of_lane(sc, base, count, T);\n"
+      << link_near << "            work += " << 2 * NL * kSph << "u;\n"
+      << "            const u64 near = " << near_any << ";\n";
     for (const Kind& kd : kinds) {
-        o << "            {\n            u64 m = near & mp_bits(base, " << kd.lo << ", " << kd.hi << ");\n"
-             "            const int nm = __popcll(m);\n"
-             "            m = mp_drop_low(m, o0);\n"
+        o << near_of(kd)
+          << "            const int nm = os * (int)__popcll(m);\n"
              "            for (int o = o0, it = 1; o < nm; o += os, ++it) {\n"
-             "            const int l = __builtin_ctzll(m), k = base + l - " << kd.lo << ";\n"
-             "            m = mp_drop_low(m, os);\n"
-          << kd.load << env_block(kd.kind, false, kd.detail)
+          << step(kd) << kd.load << env_block(kd.kind, false, kd.detail.c_str())
           << "            const u64 hb = __ballot(hit);\n"
              "            if (mp_decides<MODE>(hb, mask) || ((it & 3) == 0 && T.stopped())) return hit;\n"
              "            live = mp_live<MODE>(hb, mask);\n            }\n            }\n";
@@ -838,19 +805,19 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     // full-evaluation costs, per kind in index order (the oracle's): spheres, boxes, cylinders,
     // capsules into pk[0..3], the per-constraint costs of States.h:205's [constraint][state] rows;
     // culled blocks contribute exact zeros, so skipping them leaves every partial sum unchanged
-    o << "    static __device__ __forceinline__ void env_cost(float* F, const SceneDev& sc, mp_f4 ob, unsigned& work, float* pk) {\n"
-      << ranges << group_prologue << "        const u64 live = ~0ull, seen = live;\n" << group_balls
+    o << "    static __device__ __forceinline__ void env_cost(float* F, const SceneDev& sc, mp_f4 ob, unsigned& work, float* pk, const Team& T) {\n"
+      << ranges << "        const u64 live = ~0ull;\n"
+         "        const int o0 = 0, os = 1, chunk = MP_WAVE;\n"
       << "        pk[0] = pk[1] = pk[2] = pk[3] = 0.0f;\n"
-         "        for (int base = 0; base < count; base += MP_WAVE) {\n"
-         "            if (base > 0) ob = mp_bound_of_lane(sc, base, count);\n"
-      << group_near << "            work += " << 2 * G * kSph << "u;\n"
-      << "            const u64 near = (" << near_any << ") & mp_bits(base, 0, count);\n";
+         "        for (int base = 0; base < count; base += chunk) {\n"
+         "            if (base > 0) ob = mp_bound_of_lane(sc, base, count, T);\n"
+      << link_near << "            work += " << 2 * NL * kSph << "u;\n"
+      << "            const u64 near = " << near_any << ";\n";
     const int row_of[4] = {1, 0, 3, 2};  // box, sphere, capsule, cylinder
     for (const Kind& kd : kinds) {
-        o << "            {\n            float part = pk[" << row_of[kd.kind] << "];\n"
-             "            for (u64 m = near & mp_bits(base, " << kd.lo << ", " << kd.hi << "); m; m &= m - 1ull) {\n"
-             "            const int l = __builtin_ctzll(m), k = base + l - " << kd.lo << ";\n"
-          << kd.load << env_block(kd.kind, true, kd.detail) << "            }\n            pk[" << row_of[kd.kind] << "] = part;\n            }\n";
+        o << near_of(kd) << "            float part = pk[" << row_of[kd.kind] << "];\n"
+             "            while (m) {\n"
+          << step(kd) << kd.load << env_block(kd.kind, true, kd.detail.c_str()) << "            }\n            pk[" << row_of[kd.kind] << "] = part;\n            }\n";
     }
     o << "        }\n    }\n";
     // joint bounds: BoundaryConstraint.cu:56-92, tolerance 1e-4 on the squared sum
