@@ -30,13 +30,13 @@ def embed_template():
             f.write(new)
 
 
-HIP_SOURCES = ["noalloc.hip"]  # sources with device code of their own, compiled by hipcc
+HIP_SOURCES = ["noalloc.hip", "roadmap_io.hip"]  # sources with device code of their own, compiled by hipcc
 OBJ_DIR = os.path.join(HERE, "_build")
 
 
 def compile_hip_objects(verbose=False):
     """hipcc -c for gfx950 of the library's own device-code sources (the no-allocation entry
-    point's scratch array); returns the object paths."""
+    point's scratch array, the roadmap's start and read-out); returns the object paths."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     objs = []
     for src in HIP_SOURCES:

@@ -192,6 +192,7 @@ int mp_shutdown(void) {
         }
         G.events.clear();
         mp::plan_release_workspaces();
+        mp::roadmap_release_storage();
         if (G.work) hipFree(G.work);
         G.work = nullptr;
         if (G.prof) hipFree(G.prof);

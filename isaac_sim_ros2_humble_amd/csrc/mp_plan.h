@@ -141,6 +141,38 @@ struct LaunchPlan {
 LaunchPlan plan_launch(int nq, mp_robot* const* robots, const mp_scene* const* scenes, const mp_rrtc_params* params,
                        int default_wave_count);
 
+// The start and goal states of a roadmap (states [ns + ng][dof], loop state [nctl]; host memory that the
+// device maps) into its arrays, one launch.
+struct RoadmapStart {
+    const float* states;
+    const int* state;
+    float* node;
+    float* gq[2];
+    int* gv[2];
+    int* vgroup;
+    int* ctl;
+    int ns, ng, dof, vcap, nctl;
+};
+void roadmap_start(const RoadmapStart& a, hipStream_t s);
+// A roadmap of nv vertices, ne edges and n members laid out as the caller reads it, into host memory
+// that the device maps, one launch.
+struct RoadmapPack {
+    const float* node;
+    const int* vgroup;
+    const int* ea;
+    const int* eb;
+    const float* ew;
+    const int* gv[2];
+    int nv, ne, n[2], dof, vcap;
+    float* vertices;
+    int* groups;
+    int* edges;
+    float* weights;
+    int* members[2];
+};
+void roadmap_pack(const RoadmapPack& a, hipStream_t s);
+void roadmap_release_storage();  // frees the kept storage of destroyed roadmaps
+
 // The per-device address of the no-allocation entry point's scratch array, looked up once per
 // device with that device current (called by mp_init).
 void noalloc_setup(int device);

@@ -6,6 +6,8 @@
 // run out of room.
 #include <algorithm>
 #include <cstring>
+#include <mutex>
+#include <vector>
 
 #include "mp_plan.h"
 
@@ -50,46 +52,129 @@ float i2f(int i) {
     return f;
 }
 
+// What a roadmap lives in: one device allocation with its arrays, one host allocation that the device maps
+// (loop state, then the start and goal states or the roadmap being read out) and its events.  Destroyed
+// roadmaps leave it to the next one.  With 15 allocations, 18 copies to fill the arrays and 17 to read them,
+// a roadmap of three passes (FR3, 60 samples each, 20 spheres) took 135 us to create, 755 us to read (the
+// passes' own 150 us among them) and 87 us to destroy; four such from creation to the graph read
+// back: 2.50 -> 0.93 ms.
+struct Storage {
+    int device = -1;
+    char* dev = nullptr;
+    size_t dev_bytes = 0;
+    char* host = nullptr;
+    char* host_dev = nullptr;  // the device's address of host
+    size_t host_bytes = 0;
+    hipEvent_t ev[kDepth] = {};
+};
+constexpr size_t kStateBytes = 256;             // loop state at the head of the host allocation
+constexpr size_t kHostBytes = 256 << 10;        // host allocation of a new roadmap, unless it needs more
+constexpr size_t kKeep = 4, kKeepBytes = 8 << 20;  // storage kept: so many, each allocation up to so large
+std::mutex g_mu;                                // guards g_kept
+std::vector<Storage> g_kept;
+
+void host_alloc(Storage& st, size_t bytes) {
+    MP_HIP(hipHostMalloc((void**)&st.host, bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    st.host_bytes = bytes;
+    MP_HIP(hipHostGetDevicePointer((void**)&st.host_dev, st.host, 0));
+}
+
+void free_storage(Storage& st) {
+    if (st.dev) hipFree(st.dev);
+    if (st.host) hipHostFree(st.host);
+    for (auto& e : st.ev)
+        if (e) hipEventDestroy(e);
+    st = Storage();
+}
+
+// Kept storage with room for the sizes, else new.  `st` is the caller's to free also when this throws.
+void take_storage(Storage& st, size_t dev_bytes, size_t host_bytes) {
+    int device = 0;
+    MP_HIP(hipGetDevice(&device));
+    {
+        std::lock_guard<std::mutex> g(g_mu);
+        for (size_t i = 0; i < g_kept.size(); i++)
+            if (g_kept[i].device == device && g_kept[i].dev_bytes >= dev_bytes && g_kept[i].host_bytes >= host_bytes) {
+                st = g_kept[i];
+                g_kept.erase(g_kept.begin() + (long)i);
+                return;
+            }
+    }
+    st.device = device;
+    MP_HIP(hipMalloc((void**)&st.dev, dev_bytes));
+    st.dev_bytes = dev_bytes;
+    host_alloc(st, std::max(host_bytes, kHostBytes));
+    for (auto& e : st.ev) MP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+}
+
+// Keeps whole storage that no work uses any more (the caller has waited for the stream) or frees it.
+void give_back(Storage& st) {
+    if (st.dev && st.host_dev && st.ev[kDepth - 1] && st.dev_bytes <= kKeepBytes && st.host_bytes <= kKeepBytes) {
+        std::lock_guard<std::mutex> g(g_mu);
+        if (g_kept.size() < kKeep) {
+            g_kept.push_back(st);
+            st = Storage();
+            return;
+        }
+    }
+    free_storage(st);
+}
+
+// Bytes of a roadmap's arrays; sets g's pointers into `base` when there is one.  Every array starts at a
+// multiple of 256 bytes.
+size_t place(RoadmapDevHost& g, char* base, size_t vcap, size_t ecap) {
+    size_t at = 0;
+    auto put = [&](auto*& p, size_t n) {
+        if (base) p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + at);
+        at += (n * sizeof(*p) + 255) & ~(size_t)255;
+    };
+    const size_t dof = (size_t)g.dof, k = (size_t)g.k;
+    put(g.ctl, kNctl);
+    put(g.smp, k * dof);
+    put(g.nn, 3 * k);
+    put(g.ok, 2 * k);
+    put(g.len, 2 * k);
+    put(g.freed, k);
+    put(g.node, dof * vcap);
+    for (int s = 0; s < 2; s++) {
+        put(g.gq[s], dof * vcap);
+        put(g.gv[s], vcap);
+    }
+    put(g.vgroup, vcap);
+    put(g.ea, ecap);
+    put(g.eb, ecap);
+    put(g.ew, ecap);
+    if (base) {
+        g.vcap = (int)vcap;
+        g.ecap = (int)ecap;
+    }
+    return at;
+}
+
 }  // namespace
+
+namespace mp {
+
+void roadmap_release_storage() {
+    std::lock_guard<std::mutex> g(g_mu);
+    for (Storage& st : g_kept) free_storage(st);
+    g_kept.clear();
+}
+
+}  // namespace mp
 
 struct mp_roadmap {
     mp_robot* robot = nullptr;
     const mp_scene* scene = nullptr;
     RoadmapDevHost g{};
-    int* mirror_h = nullptr;   // host-mapped loop state
-    hipEvent_t ev[kDepth] = {};
+    Storage mem;
+    int* mirror_h = nullptr;   // host-mapped loop state: equal to ctl when no pass is in flight
     long long enqueued = 0, completed = 0;  // passes enqueued / known finished
     hipFunction_t f_sample = nullptr, f_edges = nullptr, f_commit = nullptr;
 
-    void alloc(int vcap, int ecap);
-    void release();
     void grow(int need_v, int need_e);
     void wait_all();
 };
-
-void mp_roadmap::alloc(int vcap, int ecap) {
-    const int dof = g.dof;
-    g.vcap = vcap;
-    g.ecap = ecap;
-    MP_HIP(hipMalloc(&g.node, (size_t)dof * vcap * sizeof(float)));
-    MP_HIP(hipMalloc(&g.vgroup, (size_t)vcap * sizeof(int)));
-    for (int s = 0; s < 2; s++) {
-        MP_HIP(hipMalloc(&g.gq[s], (size_t)dof * vcap * sizeof(float)));
-        MP_HIP(hipMalloc(&g.gv[s], (size_t)vcap * sizeof(int)));
-    }
-    MP_HIP(hipMalloc(&g.ea, (size_t)ecap * sizeof(int)));
-    MP_HIP(hipMalloc(&g.eb, (size_t)ecap * sizeof(int)));
-    MP_HIP(hipMalloc(&g.ew, (size_t)ecap * sizeof(float)));
-}
-
-void mp_roadmap::release() {
-    void* ps[] = {g.node, g.vgroup, g.gq[0], g.gq[1], g.gv[0], g.gv[1], g.ea, g.eb, g.ew};
-    for (void* p : ps)
-        if (p) hipFree(p);
-    g.node = nullptr;
-    g.vgroup = g.gv[0] = g.gv[1] = g.ea = g.eb = nullptr;
-    g.gq[0] = g.gq[1] = g.ew = nullptr;
-}
 
 void mp_roadmap::wait_all() {
     MP_HIP(hipStreamSynchronize(mp::lib_stream()));
@@ -105,31 +190,39 @@ void mp_roadmap::grow(int need_v, int need_e) {
     if (vcap == g.vcap && ecap == g.ecap) return;
     wait_all();
     hipStream_t s = mp::lib_stream();
-    int ctl[kNctl];
-    MP_HIP(hipMemcpy(ctl, g.ctl, sizeof(ctl), hipMemcpyDeviceToHost));
-    RoadmapDevHost old = g;
-    g.node = nullptr;
-    g.vgroup = g.gv[0] = g.gv[1] = g.ea = g.eb = nullptr;
-    g.gq[0] = g.gq[1] = g.ew = nullptr;
-    alloc(vcap, ecap);
+    const volatile int* ctl = mirror_h;
+    const RoadmapDevHost old = g;
+    const size_t bytes = place(g, nullptr, vcap, ecap);
+    char* block = nullptr;
+    MP_HIP(hipMalloc((void**)&block, bytes));
+    place(g, block, vcap, ecap);
+    char* const old_block = mem.dev;
+    mem.dev = block;
+    mem.dev_bytes = bytes;
     const int dof = g.dof, nv = ctl[NV], ne = ctl[NE], n1 = ctl[G1], n2 = ctl[G2];
-    for (int j = 0; j < dof; j++) {
-        MP_HIP(hipMemcpyAsync(g.node + (size_t)j * vcap, old.node + (size_t)j * old.vcap, (size_t)nv * 4,
-                              hipMemcpyDeviceToDevice, s));
-        MP_HIP(hipMemcpyAsync(g.gq[0] + (size_t)j * vcap, old.gq[0] + (size_t)j * old.vcap, (size_t)n1 * 4,
-                              hipMemcpyDeviceToDevice, s));
-        MP_HIP(hipMemcpyAsync(g.gq[1] + (size_t)j * vcap, old.gq[1] + (size_t)j * old.vcap, (size_t)n2 * 4,
-                              hipMemcpyDeviceToDevice, s));
+    auto copy = [&](void* to, const void* from, int n) {
+        MP_HIP(hipMemcpyAsync(to, from, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
+    };
+    try {
+        copy(g.ctl, old.ctl, kNctl);
+        for (int j = 0; j < dof; j++) {
+            copy(g.node + (size_t)j * vcap, old.node + (size_t)j * old.vcap, nv);
+            copy(g.gq[0] + (size_t)j * vcap, old.gq[0] + (size_t)j * old.vcap, n1);
+            copy(g.gq[1] + (size_t)j * vcap, old.gq[1] + (size_t)j * old.vcap, n2);
+        }
+        copy(g.vgroup, old.vgroup, nv);
+        copy(g.gv[0], old.gv[0], n1);
+        copy(g.gv[1], old.gv[1], n2);
+        copy(g.ea, old.ea, ne);
+        copy(g.eb, old.eb, ne);
+        copy(g.ew, old.ew, ne);
+        MP_HIP(hipStreamSynchronize(s));
+    } catch (...) {
+        hipStreamSynchronize(s);
+        hipFree(old_block);
+        throw;
     }
-    MP_HIP(hipMemcpyAsync(g.vgroup, old.vgroup, (size_t)nv * 4, hipMemcpyDeviceToDevice, s));
-    MP_HIP(hipMemcpyAsync(g.gv[0], old.gv[0], (size_t)n1 * 4, hipMemcpyDeviceToDevice, s));
-    MP_HIP(hipMemcpyAsync(g.gv[1], old.gv[1], (size_t)n2 * 4, hipMemcpyDeviceToDevice, s));
-    MP_HIP(hipMemcpyAsync(g.ea, old.ea, (size_t)ne * 4, hipMemcpyDeviceToDevice, s));
-    MP_HIP(hipMemcpyAsync(g.eb, old.eb, (size_t)ne * 4, hipMemcpyDeviceToDevice, s));
-    MP_HIP(hipMemcpyAsync(g.ew, old.ew, (size_t)ne * 4, hipMemcpyDeviceToDevice, s));
-    MP_HIP(hipStreamSynchronize(s));
-    void* ps[] = {old.node, old.vgroup, old.gq[0], old.gq[1], old.gv[0], old.gv[1], old.ea, old.eb, old.ew};
-    for (void* p : ps) hipFree(p);
+    hipFree(old_block);
 }
 
 extern "C" {
@@ -158,43 +251,24 @@ int mp_roadmap_create(mp_robot* robot, const mp_scene* scene, const float* start
         int vcap = 4096;
         while (vcap < nv0 + kDepth * 2 * g.k) vcap *= 2;
         try {
-            rm->alloc(vcap, 2 * vcap);
-            MP_HIP(hipMalloc(&g.smp, (size_t)g.k * dof * sizeof(float)));
-            MP_HIP(hipMalloc(&g.nn, (size_t)3 * g.k * sizeof(int)));
-            MP_HIP(hipMalloc(&g.ok, (size_t)2 * g.k));
-            MP_HIP(hipMalloc(&g.len, (size_t)2 * g.k * sizeof(float)));
-            MP_HIP(hipMalloc(&g.freed, (size_t)g.k));
-            MP_HIP(hipMalloc(&g.ctl, kNctl * sizeof(int)));
-            MP_HIP(hipHostMalloc(&rm->mirror_h, kNctl * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
-            MP_HIP(hipHostGetDevicePointer((void**)&g.mirror, rm->mirror_h, 0));
-            for (auto& e : rm->ev) MP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            const size_t state_floats = (size_t)nv0 * dof;
+            take_storage(rm->mem, place(g, nullptr, vcap, 2 * vcap), kStateBytes + state_floats * sizeof(float));
+            place(g, rm->mem.dev, vcap, 2 * vcap);
+            rm->mirror_h = reinterpret_cast<int*>(rm->mem.host);
+            g.mirror = reinterpret_cast<int*>(rm->mem.host_dev);
             // the start and goal states: vertices, and the first members of their groups
-            std::vector<float> soa((size_t)dof * nv0);
-            std::vector<int> grp(nv0), ids(nv0);
-            for (int v = 0; v < nv0; v++) {
-                const float* q = v < ns ? starts + (size_t)v * dof : goals + (size_t)(v - ns) * dof;
-                for (int j = 0; j < dof; j++) soa[(size_t)j * nv0 + v] = q[j];
-                grp[v] = v < ns ? 1 : 2;
-                ids[v] = v;
-            }
-            hipStream_t s = mp::lib_stream();
-            for (int j = 0; j < dof; j++) {
-                MP_HIP(hipMemcpyAsync(g.node + (size_t)j * vcap, &soa[(size_t)j * nv0], (size_t)nv0 * 4, hipMemcpyHostToDevice, s));
-                MP_HIP(hipMemcpyAsync(g.gq[0] + (size_t)j * vcap, &soa[(size_t)j * nv0], (size_t)ns * 4, hipMemcpyHostToDevice, s));
-                MP_HIP(hipMemcpyAsync(g.gq[1] + (size_t)j * vcap, &soa[(size_t)j * nv0 + ns], (size_t)ng * 4,
-                                      hipMemcpyHostToDevice, s));
-            }
-            MP_HIP(hipMemcpyAsync(g.vgroup, grp.data(), (size_t)nv0 * 4, hipMemcpyHostToDevice, s));
-            MP_HIP(hipMemcpyAsync(g.gv[0], ids.data(), (size_t)ns * 4, hipMemcpyHostToDevice, s));
-            MP_HIP(hipMemcpyAsync(g.gv[1], ids.data() + ns, (size_t)ng * 4, hipMemcpyHostToDevice, s));
+            float* states = reinterpret_cast<float*>(rm->mem.host + kStateBytes);
+            std::memcpy(states, starts, (size_t)ns * dof * sizeof(float));
+            std::memcpy(states + (size_t)ns * dof, goals, (size_t)ng * dof * sizeof(float));
             int ctl[kNctl] = {0};
             ctl[NV] = nv0;
             ctl[G1] = ns;
             ctl[G2] = ng;
             ctl[TRAVEL1] = ctl[TRAVEL2] = f2i(max_travel_distance);
-            MP_HIP(hipMemcpyAsync(g.ctl, ctl, sizeof(ctl), hipMemcpyHostToDevice, s));
             std::memcpy(rm->mirror_h, ctl, sizeof(ctl));
-            MP_HIP(hipStreamSynchronize(s));
+            mp::roadmap_start({reinterpret_cast<const float*>(rm->mem.host_dev + kStateBytes), g.mirror, g.node,
+                               {g.gq[0], g.gq[1]}, {g.gv[0], g.gv[1]}, g.vgroup, g.ctl, ns, ng, dof, vcap, kNctl},
+                              mp::lib_stream());
             mp::Module& mod = *robot->module;
             rm->f_sample = mod.fn("mp_rm_sample_0");
             rm->f_edges = mod.fn("mp_rm_edges_0");
@@ -213,7 +287,7 @@ int mp_roadmap_iterate(mp_roadmap* rm, int* solved) {
         RoadmapDevHost& g = rm->g;
         hipStream_t s = mp::lib_stream();
         if (rm->enqueued - rm->completed >= kDepth) {  // keep at most kDepth passes in flight
-            MP_HIP(hipEventSynchronize(rm->ev[rm->completed % kDepth]));
+            MP_HIP(hipEventSynchronize(rm->mem.ev[rm->completed % kDepth]));
             rm->completed++;
         }
         volatile int* m = rm->mirror_h;
@@ -242,7 +316,7 @@ int mp_roadmap_iterate(mp_roadmap* rm, int* solved) {
         mp::launch(rm->f_sample, 1, kMaxK, s, a1, nullptr);
         mp::launch(rm->f_edges, (unsigned)((2 * g.k + 3) / 4), 256, s, a2, "rrg");
         mp::launch(rm->f_commit, 1, 64, s, a3, nullptr);
-        MP_HIP(hipEventRecord(rm->ev[rm->enqueued % kDepth], s));
+        MP_HIP(hipEventRecord(rm->mem.ev[rm->enqueued % kDepth], s));
         rm->enqueued++;
         *solved = 0;
     });
@@ -252,8 +326,7 @@ int mp_roadmap_info_get(mp_roadmap* rm, mp_roadmap_info* info) {
     return mp::guard_call([&] {
         if (!rm || !info) throw Error(MP_E_INVALID, "bad arguments");
         rm->wait_all();
-        int c[kNctl];
-        MP_HIP(hipMemcpy(c, rm->g.ctl, sizeof(c), hipMemcpyDeviceToHost));
+        const volatile int* c = rm->mirror_h;
         info->solved = c[SOLVED];
         info->passes = c[PASS];
         info->loop_index = c[T];
@@ -272,43 +345,46 @@ int mp_roadmap_read(mp_roadmap* rm, float* vertices, int* groups, int* edges, fl
         if (!rm) throw Error(MP_E_INVALID, "null roadmap");
         rm->wait_all();
         const RoadmapDevHost& g = rm->g;
-        int c[kNctl];
-        MP_HIP(hipMemcpy(c, g.ctl, sizeof(c), hipMemcpyDeviceToHost));
-        const int nv = c[NV], ne = c[NE], dof = g.dof;
-        if (vertices && nv > 0) {
-            std::vector<float> soa((size_t)dof * nv);
-            for (int j = 0; j < dof; j++)
-                MP_HIP(hipMemcpy(&soa[(size_t)j * nv], g.node + (size_t)j * g.vcap, (size_t)nv * 4, hipMemcpyDeviceToHost));
-            for (int v = 0; v < nv; v++)
-                for (int j = 0; j < dof; j++) vertices[(size_t)v * dof + j] = soa[(size_t)j * nv + v];
-        }
-        if (groups && nv > 0) MP_HIP(hipMemcpy(groups, g.vgroup, (size_t)nv * 4, hipMemcpyDeviceToHost));
-        if (edges && ne > 0) {
-            std::vector<int> a(ne), b(ne);
-            MP_HIP(hipMemcpy(a.data(), g.ea, (size_t)ne * 4, hipMemcpyDeviceToHost));
-            MP_HIP(hipMemcpy(b.data(), g.eb, (size_t)ne * 4, hipMemcpyDeviceToHost));
-            for (int e = 0; e < ne; e++) {
-                edges[2 * e] = a[e];
-                edges[2 * e + 1] = b[e];
+        const volatile int* c = rm->mirror_h;
+        const size_t nv = (size_t)c[NV], ne = (size_t)c[NE], n1 = (size_t)c[G1], n2 = (size_t)c[G2], dof = (size_t)g.dof;
+        const size_t words[6] = {nv * dof, nv, 2 * ne, ne, n1, n2};
+        size_t at[7] = {kStateBytes};
+        for (int i = 0; i < 6; i++) at[i + 1] = at[i] + words[i] * 4;
+        if (at[6] > rm->mem.host_bytes) {  // the loop state moves along
+            Storage old = rm->mem;
+            rm->mem.host = rm->mem.host_dev = nullptr;
+            try {
+                host_alloc(rm->mem, at[6] + at[6] / 2);
+            } catch (...) {
+                if (rm->mem.host) hipHostFree(rm->mem.host);
+                rm->mem = old;
+                throw;
             }
+            std::memcpy(rm->mem.host, old.host, kStateBytes);
+            hipHostFree(old.host);
+            rm->mirror_h = reinterpret_cast<int*>(rm->mem.host);
+            rm->g.mirror = reinterpret_cast<int*>(rm->mem.host_dev);
         }
-        if (weights && ne > 0) MP_HIP(hipMemcpy(weights, g.ew, (size_t)ne * 4, hipMemcpyDeviceToHost));
-        if (start_members && c[G1] > 0) MP_HIP(hipMemcpy(start_members, g.gv[0], (size_t)c[G1] * 4, hipMemcpyDeviceToHost));
-        if (goal_members && c[G2] > 0) MP_HIP(hipMemcpy(goal_members, g.gv[1], (size_t)c[G2] * 4, hipMemcpyDeviceToHost));
+        char* const d = rm->mem.host_dev;
+        hipStream_t s = mp::lib_stream();
+        mp::roadmap_pack({g.node, g.vgroup, g.ea, g.eb, g.ew, {g.gv[0], g.gv[1]}, (int)nv, (int)ne, {(int)n1, (int)n2}, g.dof, g.vcap,
+                          (float*)(d + at[0]), (int*)(d + at[1]), (int*)(d + at[2]), (float*)(d + at[3]),
+                          {(int*)(d + at[4]), (int*)(d + at[5])}},
+                         s);
+        MP_HIP(hipStreamSynchronize(s));
+        void* const to[6] = {vertices, groups, edges, weights, start_members, goal_members};
+        for (int i = 0; i < 6; i++)
+            if (to[i] && words[i]) std::memcpy(to[i], rm->mem.host + at[i], words[i] * 4);
     });
 }
 
 int mp_roadmap_destroy(mp_roadmap* rm) {
     return mp::guard_call([&] {
         if (!rm) return;
-        if (mp::lib_stream()) hipStreamSynchronize(mp::lib_stream());
-        rm->release();
-        void* ps[] = {rm->g.smp, rm->g.nn, rm->g.ok, rm->g.len, rm->g.freed, rm->g.ctl};
-        for (void* p : ps)
-            if (p) hipFree(p);
-        if (rm->mirror_h) hipHostFree(rm->mirror_h);
-        for (auto& e : rm->ev)
-            if (e) hipEventDestroy(e);
+        if (mp::lib_stream() && hipStreamSynchronize(mp::lib_stream()) == hipSuccess)
+            give_back(rm->mem);
+        else
+            free_storage(rm->mem);
         delete rm;
     });
 }

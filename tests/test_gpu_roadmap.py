@@ -85,3 +85,33 @@ def test_roadmap_grows_and_halves(rng):
     # the oracle's run halved the goal side's travel distance on the way (the shell blocks it)
     part = oracle.rrg(oracle.OracleRobot(m), oracle.OracleScene(scene), s, g, 256, 1.0, 0.02, 5, 0, max_passes=2)
     assert part["travel_goal"] == np.float32(0.5) and part["loop_index"] == 3
+
+
+def test_roadmaps_one_after_another_and_together(fr3, orc_fr3):
+    """Roadmaps take over the storage of destroyed ones: several starts and goals, then fewer, then two at
+    once, then one larger than the storage kept, each equal to the oracle's and read twice alike."""
+    rng = np.random.default_rng(3)
+    scene = workloads.random_scene(rng, 20, *workloads.workspace(fr3))
+    r, ns = robot(fr3), native.Scene(scene)
+    q = workloads.uniform_configs(fr3, 40000, rng)
+    q = q[native.check_states(r, ns, q).astype(bool)]
+    osc = oracle.OracleScene(scene)
+
+    def make(a, b, seed):
+        return native.Roadmap(r, ns, q[:a], q[a:a + b], samples_per_iteration=33, max_travel_distance=1.5, resolution=0.02, seed=seed)
+
+    def finish(rm, a, b, seed):
+        for _ in range(4):
+            if rm.iterate():
+                break
+        got, again = rm.read(), rm.read()
+        rm.close()
+        want = oracle.rrg(orc_fr3, osc, q[:a], q[a:a + b], 33, 1.5, 0.02, seed, 0, max_passes=got["passes"], vcap=1 << 15)
+        assert_same(got, want)
+        assert_same(again, want)
+
+    for a, b, seed in ((5, 3, 1), (1, 1, 2), (2, 64, 3), (5000, 4000, 4), (1, 2, 5)):
+        finish(make(a, b, seed), a, b, seed)
+    first, second = make(3, 1, 6), make(1, 4, 7)
+    finish(second, 1, 4, 7)
+    finish(first, 3, 1, 6)
