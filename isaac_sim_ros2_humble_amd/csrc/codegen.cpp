@@ -597,122 +597,134 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     // kind: 0 box, 1 sphere, 2 capsule, 3 cylinder.  The obstacle parameters are named
     // m0..m11 lo{x,y,z} hi{x,y,z} (box), ox oy oz orad (sphere), x1 y1 z1 xv yv zv rdv crad
     // (capsule), m0..m11 crad hh (cylinder) in the generated loops.
-    auto env_block = [&](int kind, bool cost, const char* detail) {
+    const int tests[4] = {kBox, kSph, kCap, kCyl};
+    V mm[12];
+    for (int i = 0; i < 12; i++) mm[i] = V{false, 0.0f, "m" + std::to_string(i)};
+    // whether link k's bounding sphere may touch the obstacle
+    auto link_reaches = [&](Emitter& X, int kind, int k) {
+        const float Rm = (float)(SL[k].R + kCullMargin);
+        V b[3];
+        link_centre(X, k, b);
+        std::string cond;
+        if (kind == 0 || kind == 3) {
+            V l[3];
+            for (int a = 0; a < 3; a++) l[a] = X.row(mm[4 * a], b[0], mm[4 * a + 1], b[1], mm[4 * a + 2], b[2], mm[4 * a + 3]);
+            if (kind == 0) {
+                const char* lo[3] = {"lox", "loy", "loz"};
+                const char* hi[3] = {"hix", "hiy", "hiz"};
+                V d[3];
+                for (int a = 0; a < 3; a++)
+                    d[a] = X.tmp(X.ref(l[a]) + " - fminf(fmaxf(" + X.ref(l[a]) + ", " + lo[a] + "), " + hi[a] + ")");
+                V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
+                cond = X.ref(d2) + " < " + lit(Rm * Rm);
+            } else {
+                cond = "mp_cyl_near(" + X.ref(l[0]) + ", " + X.ref(l[1]) + ", " + X.ref(l[2]) + ", crad, hh, " + lit(Rm) + ")";
+            }
+        } else if (kind == 1) {
+            V d[3] = {X.sub(b[0], V{false, 0, "ox"}), X.sub(b[1], V{false, 0, "oy"}), X.sub(b[2], V{false, 0, "oz"})};
+            V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
+            V sr = X.tmp(lit(Rm) + " + orad");
+            cond = X.ref(d2) + " < " + X.ref(sr) + " * " + X.ref(sr);
+        } else {
+            V d2 = X.tmp("mp_cap_d2(" + X.ref(b[0]) + ", " + X.ref(b[1]) + ", " + X.ref(b[2]) + ", x1, y1, z1, xv, yv, zv, rdv)");
+            V sr = X.tmp(lit(Rm) + " + crad");
+            cond = X.ref(d2) + " < " + X.ref(sr) + " * " + X.ref(sr);
+        }
+        return cond;
+    };
+    // link k's spheres against the obstacle, into `hit` (or the penetrations into `part`); among:
+    // what is ANDed to the ballots that decide for the wave
+    auto link_spheres = [&](Emitter& X, int kind, bool cost, int k, const char* among) {
+        const SphereLink& L = SL[k];
+        // spheres and capsules: contact <=> d2 < (r+R)^2 and sqrtf(d2) < r+R (the cost
+        // (r+R) - sqrtf(d2) is then > 0); a fast test with a 1e-6 relative margin, then the
+        // exact test for lanes in the thin band below the threshold
+        const bool banded = (kind == 1 || kind == 2) && !cost;
+        if (banded) X.os << "                bool band = false;\n";
+        std::vector<std::string> d2n, srn;
+        for (int s : L.spheres) {
+            V c[3];
+            centre(X, s, c);
+            float r = m.sphere_r[s];
+            if (kind == 0) {
+                V l[3];
+                for (int a = 0; a < 3; a++) l[a] = X.row(mm[4 * a], c[0], mm[4 * a + 1], c[1], mm[4 * a + 2], c[2], mm[4 * a + 3]);
+                const char* lo[3] = {"lox", "loy", "loz"};
+                const char* hi[3] = {"hix", "hiy", "hiz"};
+                V d[3];
+                for (int a = 0; a < 3; a++)
+                    d[a] = X.tmp(X.ref(l[a]) + " - fminf(fmaxf(" + X.ref(l[a]) + ", " + lo[a] + "), " + hi[a] + ")");
+                V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
+                if (cost)
+                    X.os << "                if (__ballot(" << X.ref(d2) << " < " << lit(r * r) << "))\n                    part += "
+                         << X.ref(d2) << " < " << lit(r * r) << " ? " << lit(r) << " - __builtin_sqrtf(" << X.ref(d2)
+                         << ") : 0.0f;\n";
+                else
+                    X.os << "                hit |= " << X.ref(d2) << " < " << lit(boxte[s]) << ";\n";
+            } else if (kind == 1) {
+                V d[3] = {X.sub(c[0], V{false, 0, "ox"}), X.sub(c[1], V{false, 0, "oy"}), X.sub(c[2], V{false, 0, "oz"})};
+                V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
+                V sr = X.tmp(lit(r) + " + orad");
+                if (cost) {
+                    X.os << "                if (__ballot(" << X.ref(d2) << " < " << X.ref(sr) << " * " << X.ref(sr)
+                         << "))\n                    part += " << X.ref(d2) << " < " << X.ref(sr) << " * " << X.ref(sr)
+                         << " ? fmaxf(0.0f, " << X.ref(sr) << " - __builtin_sqrtf(" << X.ref(d2) << ")) : 0.0f;\n";
+                } else {
+                    V T2 = X.tmp(X.ref(sr) + " * " + X.ref(sr));
+                    X.os << "                hit |= " << X.ref(d2) << " < " << X.ref(T2) << " * 0.999999f;\n";
+                    X.os << "                band |= " << X.ref(d2) << " < " << X.ref(T2) << ";\n";
+                    d2n.push_back(X.ref(d2));
+                    srn.push_back(X.ref(sr));
+                }
+            } else if (kind == 2) {
+                V d2 = X.tmp("mp_cap_d2(" + X.ref(c[0]) + ", " + X.ref(c[1]) + ", " + X.ref(c[2]) + ", x1, y1, z1, xv, yv, zv, rdv)");
+                V rs = X.tmp(lit(r) + " + crad");
+                if (cost) {
+                    X.os << "                if (__ballot(" << X.ref(d2) << " < " << X.ref(rs) << " * " << X.ref(rs)
+                         << "))\n                    part += " << X.ref(d2) << " < " << X.ref(rs) << " * " << X.ref(rs)
+                         << " ? fmaxf(0.0f, " << X.ref(rs) << " - __builtin_sqrtf(" << X.ref(d2) << ")) : 0.0f;\n";
+                } else {
+                    V T2 = X.tmp(X.ref(rs) + " * " + X.ref(rs));
+                    X.os << "                hit |= " << X.ref(d2) << " < " << X.ref(T2) << " * 0.999999f;\n";
+                    X.os << "                band |= " << X.ref(d2) << " < " << X.ref(T2) << ";\n";
+                    d2n.push_back(X.ref(d2));
+                    srn.push_back(X.ref(rs));
+                }
+            } else {
+                V l[3];
+                for (int a = 0; a < 3; a++) l[a] = X.row(mm[4 * a], c[0], mm[4 * a + 1], c[1], mm[4 * a + 2], c[2], mm[4 * a + 3]);
+                // the distance takes two square roots: only when some lane's sphere is near
+                X.os << "                if (__ballot(mp_cyl_near(" << X.ref(l[0]) << ", " << X.ref(l[1]) << ", " << X.ref(l[2])
+                     << ", crad, hh, " << lit(r) << "))" << among << ") {\n";
+                V sdf = X.tmp("mp_cyl_sdf(" + X.ref(l[0]) + ", " + X.ref(l[1]) + ", " + X.ref(l[2]) + ", crad, hh)");
+                if (cost)
+                    X.os << "                const float pen = " << lit(r) << " - " << X.ref(sdf)
+                         << "; part += pen > 0.0f ? pen : 0.0f; }\n";
+                else
+                    X.os << "                hit |= " << X.ref(sdf) << " < " << lit(r) << "; }\n";
+            }
+        }
+        if (banded) {
+            X.os << "                if (__ballot(band && !hit)) {\n";
+            for (size_t t = 0; t < d2n.size(); t++)
+                X.os << "                    hit |= (" << d2n[t] << " < " << srn[t] << " * " << srn[t] << ") && (__builtin_sqrtf("
+                     << d2n[t] << ") < " << srn[t] << ");\n";
+            X.os << "                }\n";
+        }
+    };
+    // one obstacle against every link; masked: only the links whose wave mask lm has it
+    auto env_block = [&](int kind, bool cost, const char* detail, bool masked = true) {
         Emitter X;
-        V mm[12];
-        for (int i = 0; i < 12; i++) mm[i] = V{false, 0.0f, "m" + std::to_string(i)};
         X.os << pin << detail;
         for (int k = 0; k < NL; k++) {
-            const SphereLink& L = SL[k];
-            float Rm = (float)(L.R + kCullMargin);
-            int n = (int)L.spheres.size();
-            X.os << "            if ((lm" << k << " >> l) & 1ull) {\n";
-            V b[3];
-            link_centre(X, k, b);
-            std::string cond;
-            int tcost = kind == 0 ? kBox : kind == 1 ? kSph : kind == 2 ? kCap : kCyl;
-            if (kind == 0 || kind == 3) {
-                V l[3];
-                for (int a = 0; a < 3; a++) l[a] = X.row(mm[4 * a], b[0], mm[4 * a + 1], b[1], mm[4 * a + 2], b[2], mm[4 * a + 3]);
-                if (kind == 0) {
-                    const char* lo[3] = {"lox", "loy", "loz"};
-                    const char* hi[3] = {"hix", "hiy", "hiz"};
-                    V d[3];
-                    for (int a = 0; a < 3; a++)
-                        d[a] = X.tmp(X.ref(l[a]) + " - fminf(fmaxf(" + X.ref(l[a]) + ", " + lo[a] + "), " + hi[a] + ")");
-                    V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
-                    cond = X.ref(d2) + " < " + lit(Rm * Rm);
-                } else {
-                    cond = "mp_cyl_near(" + X.ref(l[0]) + ", " + X.ref(l[1]) + ", " + X.ref(l[2]) + ", crad, hh, " + lit(Rm) + ")";
-                }
-            } else if (kind == 1) {
-                V d[3] = {X.sub(b[0], V{false, 0, "ox"}), X.sub(b[1], V{false, 0, "oy"}), X.sub(b[2], V{false, 0, "oz"})};
-                V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
-                V sr = X.tmp(lit(Rm) + " + orad");
-                cond = X.ref(d2) + " < " + X.ref(sr) + " * " + X.ref(sr);
-            } else {
-                V d2 = X.tmp("mp_cap_d2(" + X.ref(b[0]) + ", " + X.ref(b[1]) + ", " + X.ref(b[2]) + ", x1, y1, z1, xv, yv, zv, rdv)");
-                V sr = X.tmp(lit(Rm) + " + crad");
-                cond = X.ref(d2) + " < " + X.ref(sr) + " * " + X.ref(sr);
-            }
+            const int n = (int)SL[k].spheres.size(), tcost = tests[kind];
+            const char* among = cost ? "" : " & live";
+            X.os << "            " << (masked ? "if ((lm" + std::to_string(k) + " >> l) & 1ull) " : std::string()) << "{\n";
+            const std::string cond = link_reaches(X, kind, k);
             X.os << "            work += " << tcost << "u;\n";
-            X.os << "            if (__ballot(" << cond << ")" << (cost ? "" : " & live") << ") {\n";
+            X.os << "            if (__ballot(" << cond << ")" << among << ") {\n";
             X.os << "                work += " << n * (kXform + tcost) << "u;\n";
-            // spheres and capsules: contact <=> d2 < (r+R)^2 and sqrtf(d2) < r+R (the cost
-            // (r+R) - sqrtf(d2) is then > 0); a fast test with a 1e-6 relative margin, then the
-            // exact test for lanes in the thin band below the threshold
-            const bool banded = (kind == 1 || kind == 2) && !cost;
-            if (banded) X.os << "                bool band = false;\n";
-            std::vector<std::string> d2n, srn;
-            for (int s : L.spheres) {
-                V c[3];
-                centre(X, s, c);
-                float r = m.sphere_r[s];
-                if (kind == 0) {
-                    V l[3];
-                    for (int a = 0; a < 3; a++) l[a] = X.row(mm[4 * a], c[0], mm[4 * a + 1], c[1], mm[4 * a + 2], c[2], mm[4 * a + 3]);
-                    const char* lo[3] = {"lox", "loy", "loz"};
-                    const char* hi[3] = {"hix", "hiy", "hiz"};
-                    V d[3];
-                    for (int a = 0; a < 3; a++)
-                        d[a] = X.tmp(X.ref(l[a]) + " - fminf(fmaxf(" + X.ref(l[a]) + ", " + lo[a] + "), " + hi[a] + ")");
-                    V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
-                    if (cost)
-                        X.os << "                if (__ballot(" << X.ref(d2) << " < " << lit(r * r) << "))\n                    part += "
-                             << X.ref(d2) << " < " << lit(r * r) << " ? " << lit(r) << " - __builtin_sqrtf(" << X.ref(d2)
-                             << ") : 0.0f;\n";
-                    else
-                        X.os << "                hit |= " << X.ref(d2) << " < " << lit(boxte[s]) << ";\n";
-                } else if (kind == 1) {
-                    V d[3] = {X.sub(c[0], V{false, 0, "ox"}), X.sub(c[1], V{false, 0, "oy"}), X.sub(c[2], V{false, 0, "oz"})};
-                    V d2 = X.dot3(d[0], d[0], d[1], d[1], d[2], d[2]);
-                    V sr = X.tmp(lit(r) + " + orad");
-                    if (cost) {
-                        X.os << "                if (__ballot(" << X.ref(d2) << " < " << X.ref(sr) << " * " << X.ref(sr)
-                             << "))\n                    part += " << X.ref(d2) << " < " << X.ref(sr) << " * " << X.ref(sr)
-                             << " ? fmaxf(0.0f, " << X.ref(sr) << " - __builtin_sqrtf(" << X.ref(d2) << ")) : 0.0f;\n";
-                    } else {
-                        V T2 = X.tmp(X.ref(sr) + " * " + X.ref(sr));
-                        X.os << "                hit |= " << X.ref(d2) << " < " << X.ref(T2) << " * 0.999999f;\n";
-                        X.os << "                band |= " << X.ref(d2) << " < " << X.ref(T2) << ";\n";
-                        d2n.push_back(X.ref(d2));
-                        srn.push_back(X.ref(sr));
-                    }
-                } else if (kind == 2) {
-                    V d2 = X.tmp("mp_cap_d2(" + X.ref(c[0]) + ", " + X.ref(c[1]) + ", " + X.ref(c[2]) + ", x1, y1, z1, xv, yv, zv, rdv)");
-                    V rs = X.tmp(lit(r) + " + crad");
-                    if (cost) {
-                        X.os << "                if (__ballot(" << X.ref(d2) << " < " << X.ref(rs) << " * " << X.ref(rs)
-                             << "))\n                    part += " << X.ref(d2) << " < " << X.ref(rs) << " * " << X.ref(rs)
-                             << " ? fmaxf(0.0f, " << X.ref(rs) << " - __builtin_sqrtf(" << X.ref(d2) << ")) : 0.0f;\n";
-                    } else {
-                        V T2 = X.tmp(X.ref(rs) + " * " + X.ref(rs));
-                        X.os << "                hit |= " << X.ref(d2) << " < " << X.ref(T2) << " * 0.999999f;\n";
-                        X.os << "                band |= " << X.ref(d2) << " < " << X.ref(T2) << ";\n";
-                        d2n.push_back(X.ref(d2));
-                        srn.push_back(X.ref(rs));
-                    }
-                } else {
-                    V l[3];
-                    for (int a = 0; a < 3; a++) l[a] = X.row(mm[4 * a], c[0], mm[4 * a + 1], c[1], mm[4 * a + 2], c[2], mm[4 * a + 3]);
-                    // the distance takes two square roots: only when some lane's sphere is near
-                    X.os << "                if (__ballot(mp_cyl_near(" << X.ref(l[0]) << ", " << X.ref(l[1]) << ", " << X.ref(l[2])
-                         << ", crad, hh, " << lit(r) << "))" << (cost ? "" : " & live") << ") {\n";
-                    V sdf = X.tmp("mp_cyl_sdf(" + X.ref(l[0]) + ", " + X.ref(l[1]) + ", " + X.ref(l[2]) + ", crad, hh)");
-                    if (cost)
-                        X.os << "                const float pen = " << lit(r) << " - " << X.ref(sdf)
-                             << "; part += pen > 0.0f ? pen : 0.0f; }\n";
-                    else
-                        X.os << "                hit |= " << X.ref(sdf) << " < " << lit(r) << "; }\n";
-                }
-            }
-            if (banded) {
-                X.os << "                if (__ballot(band && !hit)) {\n";
-                for (size_t t = 0; t < d2n.size(); t++)
-                    X.os << "                    hit |= (" << d2n[t] << " < " << srn[t] << " * " << srn[t] << ") && (__builtin_sqrtf("
-                         << d2n[t] << ") < " << srn[t] << ");\n";
-                X.os << "                }\n";
-            }
+            link_spheres(X, kind, cost, k, among);
             X.os << "            }\n            }\n";
         }
         return X.os.str();
@@ -759,8 +771,9 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     std::vector<std::string> box_names = pose, cyl_names = pose;
     for (const char* f : {"lox", "loy", "loz", "hix", "hiy", "hiz"}) box_names.push_back(f);
     for (const char* f : {"crad", "hh"}) cyl_names.push_back(f);
+    const std::vector<std::string> cap_names = {"x1", "y1", "z1", "xv", "yv", "zv", "rdv", "crad"};
     const std::string box_detail = fields(box_names), cyl_detail = fields(cyl_names),
-                      cap_detail = fields({"x1", "y1", "z1", "xv", "yv", "zv", "rdv", "crad"});
+                      cap_detail = fields(cap_names);
     // the kinds' ranges in the run of bounding spheres
     const char* ranges =
         "        const int nb = mp_uniform(sc.nb), ns = mp_uniform(sc.ns), ncap = mp_uniform(sc.ncap), nc = mp_uniform(sc.nc);\n"
@@ -781,6 +794,81 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     auto step = [](const Kind& kd) {
         return "            const int l = __builtin_ctzll(m);\n            m &= m - 1ull;\n" +
                (*kd.record ? "            const float* rec = " + std::string(kd.record) + ";\n" : std::string());
+    };
+    // env_hit and env_cost for scattered states: every lane finds the obstacles near
+    // each of its own links (bits of e) and walks those, so a link's spheres are evaluated as often as the
+    // lane with the most near obstacles needs, not once per obstacle that is near any of 64 lanes.  A
+    // verdict's settled lanes leave; the costs take down the obstacles in contact (bits of touch) and then
+    // evaluate those in index order, the others' terms being exact zeros.  work counts what each lane did.
+    // Bound by the sphere tests' arithmetic and the gathers of the lanes' own records; a function of its
+    // own, as sharing the link masks with the other form spilled 42 registers (730 against 711 us for a
+    // million random FR3 states; the figures of the choice stand at mp_scattered).
+    const int row_of[4] = {1, 0, 3, 2};  // costs: box, sphere, capsule, cylinder
+    auto each_lane = [&](bool cost) {
+        const char* kind_name[4] = {"box", "sph", "cap", "cyl"};
+        const std::vector<std::string> sphere_names = {"ox", "oy", "oz", "orad"};
+        auto names_of = [&](int kind) -> const std::vector<std::string>& {
+            return kind == 0 ? box_names : kind == 1 ? sphere_names : kind == 2 ? cap_names : cyl_names;
+        };
+        auto record_of = [](int kind) {
+            return kind == 0   ? "sc.box + (base + sh + l) * MP_BOX_W"
+                   : kind == 1 ? "sc.bbox + (base + sh + l) * 4"
+                   : kind == 2 ? "sc.cap + (base + sh + l - e1) * MP_CAP_W"
+                               : "sc.cyl + (base + sh + l - e2) * MP_CYL_W";
+        };
+        std::ostringstream each;
+        each << "            ob.w = reach;\n"
+                "            mp_wave_sync();\n"
+                "            tile[threadIdx.x & (MP_WAVE - 1)] = ob;\n"
+                "            mp_wave_sync();\n"
+                "            for (int sh = 0; sh < MP_WAVE && base + sh < count; sh += 32) {\n";
+        if (cost) each << "            u32 touch = 0u;\n";
+        for (const Kind& kd : kinds)
+            each << "            const u32 m_" << kind_name[kd.kind] << " = (u32)(mp_lanes_of(base, " << kd.lo << ", " << kd.hi << ", T) >> sh);\n";
+        for (int k = 0; k < NL; k++) {
+            Emitter X;
+            X.pfx = "e" + std::to_string(k) + "_";
+            X.ind = "                ";
+            X.os << (cost ? "            {\n" : "            live = __ballot(!hit);\n            if (live) {\n")
+                 << "            const u32 near = (u32)(lm" << k << " >> sh);\n            if (near) {\n";
+            for (int e = 0; e < 12; e++)
+                if (!FV[k][e].k) X.os << "                asm volatile(\"\" : \"+v\"(" << FV[k][e].e << "));\n";
+            V b[3];
+            link_centre(X, k, b);
+            const std::string all = "mp_near_of_lane(tile + sh, near, " + lit((float)(SL[k].R + 2.0 * kCullMargin)) + ", " + X.ref(b[0]) + ", " +
+                                    X.ref(b[1]) + ", " + X.ref(b[2]) + ")";
+            X.os << "                const u32 e = " << (cost ? all + " & ~touch" : "hit ? 0u : " + all) << ";\n"
+                 << "                work += (unsigned)__popc(near) * " << kSph << "u;\n";
+            for (const Kind& kd : kinds) {
+                const std::vector<std::string>& names = names_of(kd.kind);
+                X.os << "                for (u32 m = e & m_" << kind_name[kd.kind] << "; m;) {\n                float ";
+                for (size_t f = 0; f < names.size(); f++) X.os << (f ? ", " : "") << names[f];
+                X.os << ";\n                int l;\n                bool near_link;\n                do {\n"
+                        "                l = __builtin_ctz(m);\n                m &= m - 1u;\n"
+                     << "                const float* rec = " << record_of(kd.kind) << ";\n";
+                for (size_t f = 0; f < names.size(); f++) X.os << "                " << names[f] << " = rec[" << f << "];\n";
+                const std::string cond = link_reaches(X, kd.kind, k);
+                X.os << "                near_link = " << cond << ";\n                work += " << tests[kd.kind] << "u;\n"
+                        "                } while (!near_link && m);\n                if (near_link) {\n";
+                X.os << "                work += " << (int)SL[k].spheres.size() * (kXform + tests[kd.kind]) << "u;\n";
+                if (cost) X.os << "                bool hit = false;\n";
+                link_spheres(X, kd.kind, false, k, "");
+                X.os << (cost ? "                touch |= hit ? 1u << l : 0u;\n" : "                if (hit) m = 0u;\n")
+                     << "                }\n                }\n";
+            }
+            each << X.os.str() << "            }\n            }\n";
+        }
+        if (cost)
+            for (const Kind& kd : kinds) {
+                const std::vector<std::string>& names = names_of(kd.kind);
+                each << "            if (__ballot(touch & m_" << kind_name[kd.kind] << ")) {\n            float part = pk[" << row_of[kd.kind]
+                     << "];\n            for (u32 m = touch & m_" << kind_name[kd.kind] << "; m; m &= m - 1u) {\n"
+                     << "            const int l = __builtin_ctz(m);\n            const float* rec = " << record_of(kd.kind) << ";\n";
+                for (size_t f = 0; f < names.size(); f++) each << "            const float " << names[f] << " = rec[" << f << "];\n";
+                each << env_block(kd.kind, true, "", false) << "            }\n            pk[" << row_of[kd.kind] << "] = part;\n            }\n";
+            }
+        each << "            }\n";
+        return each.str();
     };
     // The near obstacles of a kind that the wave takes: its lanes' bits, number o of the team's (o % W
     // == w).  The team's early-exit flag (an LDS read) is looked at every fourth of them.
@@ -813,13 +901,35 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
          "            if (base > 0) ob = mp_bound_of_lane(sc, base, count, T);\n"
       << link_near << "            work += " << 2 * NL * kSph << "u;\n"
       << "            const u64 near = " << near_any << ";\n";
-    const int row_of[4] = {1, 0, 3, 2};  // box, sphere, capsule, cylinder
     for (const Kind& kd : kinds) {
         o << near_of(kd) << "            float part = pk[" << row_of[kd.kind] << "];\n"
              "            while (m) {\n"
           << step(kd) << kd.load << env_block(kd.kind, true, kd.detail.c_str()) << "            }\n            pk[" << row_of[kd.kind] << "] = part;\n            }\n";
     }
     o << "        }\n    }\n";
+    const std::string each_head = std::string(ranges) + "        const Team T = mp_solo();\n        u64 live = ~0ull;\n",
+                      each_chunk = "            if (base > 0) ob = mp_bound_of_lane(sc, base, count, T);\n" + link_near +
+                                   "            work += " + std::to_string(2 * NL * kSph) + "u;\n";
+    o << "    static __device__ __forceinline__ bool env_hit_each(float* F, const SceneDev& sc, mp_f4 ob, bool hit, unsigned& work, mp_f4* tile) {\n"
+      << each_head << "        live = __ballot(!hit);\n        for (int base = 0; base < count && live; base += MP_WAVE) {\n" << each_chunk
+      << each_lane(false) << "            live = __ballot(!hit);\n        }\n        return hit;\n    }\n";
+    o << "    static __device__ __forceinline__ void env_cost_each(float* F, const SceneDev& sc, mp_f4 ob, unsigned& work, float* pk, mp_f4* tile) {\n"
+      << each_head << "        pk[0] = pk[1] = pk[2] = pk[3] = 0.0f;\n        for (int base = 0; base < count; base += MP_WAVE) {\n" << each_chunk
+      << each_lane(true) << "        }\n    }\n";
+    // whether the wave's states are scattered: the spread of the last moving link's centres
+    int last = NL - 1;
+    auto fixed = [&](int k) { return FV[k][9].k && FV[k][10].k && FV[k][11].k && FV[k][0].k; };
+    while (last >= 0 && fixed(last)) last--;
+    o << "    static __device__ __forceinline__ bool scattered(const float* F, u64 live) {\n";
+    if (last >= 0) {
+        Emitter X;
+        V b[3];
+        link_centre(X, last, b);
+        const std::string at = X.ref(b[0]) + ", " + X.ref(b[1]) + ", " + X.ref(b[2]);
+        o << X.os.str() << "        return mp_scattered(mp_half_balls(" << at << ", live));\n    }\n";
+    } else {
+        o << "        return false;\n    }\n";
+    }
     // joint bounds: BoundaryConstraint.cu:56-92, tolerance 1e-4 on the squared sum
     o << "    static __device__ __forceinline__ float bounds_acc(const float* q) {\n        float acc = 0.0f;\n";
     for (int j = 0; j < m.dof; j++) {
@@ -880,12 +990,15 @@ std::string module_source(const std::vector<const RobotModel*>& robots) {
           << "(const float* q, long long n, float* c) { mp_fk_kernel<" << R << ">(q, n, c); }\n";
         o << "extern \"C\" __global__ void __launch_bounds__(256) mp_poses_" << s
           << "(const float* q, long long n, float* p) { mp_poses_kernel<" << R << ">(q, n, p); }\n";
-        o << "extern \"C\" __global__ void __launch_bounds__(256, 2) mp_check_" << s
-          << "(const float* q, long long n, SceneDev sc, unsigned char* v, float* c, unsigned long long* w, int per_wave) { mp_check_kernel<" << R
-          << ">(q, n, sc, v, c, w, per_wave); }\n";
-        o << "extern \"C\" __global__ void __launch_bounds__(256, 2) mp_cost_" << s
-          << "(const float* q, long long n, SceneDev sc, float* c, unsigned char* v, float* parts, unsigned long long* w, int per_wave) { mp_cost_kernel<" << R
-          << ">(q, n, sc, c, v, parts, w, per_wave); }\n";
+        for (const char* each : {"", "each_"}) {
+            const char* is = *each ? ", true" : ", false";
+            o << "extern \"C\" __global__ void __launch_bounds__(256, 2) mp_check_" << each << s
+              << "(const float* q, long long n, SceneDev sc, unsigned char* v, float* c, unsigned long long* w, int per_wave) { mp_check_kernel<" << R
+              << is << ">(q, n, sc, v, c, w, per_wave); }\n";
+            o << "extern \"C\" __global__ void __launch_bounds__(256, 2) mp_cost_" << each << s
+              << "(const float* q, long long n, SceneDev sc, float* c, unsigned char* v, float* parts, unsigned long long* w, int per_wave) { mp_cost_kernel<"
+              << R << is << ">(q, n, sc, c, v, parts, w, per_wave); }\n";
+        }
         o << "extern \"C\" __global__ void __launch_bounds__(256) mp_sample_" << s
           << "(u64 seed, u64 off, long long n, float* q) { mp_sample_kernel<" << R << ">(seed, off, n, q, MP_SAMPLER_UNIFORM); }\n";
         o << "extern \"C\" __global__ void __launch_bounds__(256) mp_halton_" << s

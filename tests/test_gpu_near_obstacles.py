@@ -7,7 +7,7 @@ import pytest
 
 import oracle
 from isaac_sim_ros2_humble_amd import native, workloads
-from isaac_sim_ros2_humble_amd.scene import Scene, capsule_record, random_rotation
+from isaac_sim_ros2_humble_amd.scene import Scene, box_record, capsule_record, cylinder_record, random_rotation
 
 pytestmark = pytest.mark.gpu
 
@@ -76,3 +76,28 @@ def test_scene_update_to_fewer_obstacles(fr3, orc_fr3, robots):
         cost, v = native.state_costs(robots["fr3"], ns, q)
         assert np.array_equal(v, vo) and np.array_equal(cost, co)
         assert np.array_equal(native.check_states(robots["fr3"], ns, q), vo)
+
+
+@pytest.mark.parametrize("name,kind,count", [
+    ("fr3", "boxes", 31), ("fr3", "boxes", 65), ("fetch", "cylinders", 33), ("fr3", "capsules", 32), ("fetch", "spheres", 64),
+    ("fr3", "mixed", 97), ("fetch", "mixed", 64)])
+def test_lanes_walk_their_own_obstacles(name, kind, count, robots, request):
+    # states far from each other among obstacles within reach: nearly every link of a wave is near nearly
+    # every obstacle, the waves whose lanes take their own; 70,001 states are the last wave's remainder too
+    m = request.getfixturevalue(name)
+    rng = np.random.default_rng(count)
+
+    def pos():
+        return rng.uniform([0.45, -0.8, 0.3], [1.0, 0.8, 1.2])
+    make = {"boxes": lambda: box_record(pos(), random_rotation(rng), rng.uniform(0.01, 0.05, 3)),
+            "cylinders": lambda: cylinder_record(pos(), random_rotation(rng), rng.uniform(0.01, 0.05), rng.uniform(0.05, 0.2)),
+            "capsules": lambda: capsule_record(pos(), random_rotation(rng), rng.uniform(0.01, 0.05), rng.uniform(0.05, 0.2)),
+            "spheres": lambda: np.append(pos(), rng.uniform(0.01, 0.06))}
+    kinds = list(make) if kind == "mixed" else [kind]
+    parts = {k: np.array([make[k]() for _ in range(len(range(i, count, len(kinds))))], np.float32) for i, k in enumerate(kinds)}
+    scene = Scene(**parts)
+    assert scene.num_obstacles == count
+    q = workloads.uniform_configs(m, 70001, np.random.default_rng(count + 1))
+    vo, _, _, _ = oracle.check(request.getfixturevalue("orc_" + name), oracle.OracleScene(scene), q, nthreads=8)
+    assert 0 < vo.sum() < len(vo)
+    assert np.array_equal(native.check_states(robots[name], native.Scene(scene), q), vo)
