@@ -313,7 +313,7 @@ int mp_roadmap_iterate(mp_roadmap* rm, int* solved) {
         void* a1[] = {&g, &sv};
         void* a2[] = {&g, &sv, &work};
         void* a3[] = {&g};
-        mp::launch(rm->f_sample, 1, kMaxK, s, a1, nullptr);
+        mp::launch(rm->f_sample, (unsigned)g.k, 64, s, a1, nullptr);
         mp::launch(rm->f_edges, (unsigned)((2 * g.k + 3) / 4), 256, s, a2, "rrg");
         mp::launch(rm->f_commit, 1, 64, s, a3, nullptr);
         MP_HIP(hipEventRecord(rm->mem.ev[rm->enqueued % kDepth], s));
