@@ -705,7 +705,7 @@ def main():
     if "c2" not in a.skip:
         out["c2"] = bench_c2(robots["fr3"], models[0], max(a.steps, 3), 1)
         c2v = out["c2"]["verdict"]
-        out["roofline_c2"] = {"bound": "valu", "kernel": "mp_check_0 (2^20 FR3 configs, 64 obstacles)",
+        out["roofline_c2"] = {"bound": "valu", "kernel": "mp_check_each_0 (2^20 FR3 configs, 64 obstacles)",
                               "achieved": c2v["achieved_tflops"], "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                               "frac": c2v["achieved_tflops"] / PEAK_FP32_TFLOPS, "hbm_gbs": c2v["hbm_gbs"],
                               "hbm_frac": c2v["hbm_gbs"] / PEAK_HBM_GBS}
