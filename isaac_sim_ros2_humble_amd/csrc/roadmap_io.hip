@@ -50,18 +50,24 @@ unsigned blocks(long long elements) {
     return (unsigned)(b < 1 ? 1 : (b > 1024 ? 1024 : b));
 }
 
+// Launches kernel(a).  The launch's own status is what counts: hipGetLastError also reports what an
+// earlier call of the caller's left behind (an allocation that was refused, say).
+template <class A>
+void launch_one(void (*kernel)(A), A a, long long elements, hipStream_t s) {
+    void* args[] = {&a};
+    MP_HIP(hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(blocks(elements)), dim3(256), args, 0, s));
+}
+
 }  // namespace
 
 namespace mp {
 
 void roadmap_start(const RoadmapStart& a, hipStream_t s) {
-    start_kernel<<<blocks(((long long)a.ns + a.ng) * a.dof), 256, 0, s>>>(a);
-    MP_HIP(hipGetLastError());
+    launch_one(start_kernel, a, ((long long)a.ns + a.ng) * a.dof, s);
 }
 
 void roadmap_pack(const RoadmapPack& a, hipStream_t s) {
-    pack_kernel<<<blocks((long long)a.nv * a.dof), 256, 0, s>>>(a);
-    MP_HIP(hipGetLastError());
+    launch_one(pack_kernel, a, (long long)a.nv * a.dof, s);
 }
 
 }  // namespace mp

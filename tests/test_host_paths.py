@@ -1,0 +1,75 @@
+"""The native library's host code without a GPU: its HIP calls are answered by tests/cpp/host_hip.cpp, which
+is loaded in front of the HIP runtime in a process of its own and runs no kernels.  What is looked at:
+which calls are refused, what is allocated and what is launched."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+REPO = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C
+import sys
+sys.path.insert(0, %r)
+fake = C.CDLL(%r, mode=C.RTLD_GLOBAL)
+import numpy as np
+from isaac_sim_ros2_humble_amd import native, workloads
+from isaac_sim_ros2_humble_amd.model import load_robot
+from isaac_sim_ros2_humble_amd.scene import Scene
+
+
+class Counts(C.Structure):
+    _fields_ = [(f, C.c_longlong) for f in ("device_allocs", "device_bytes", "host_allocs", "host_bytes", "host_peak",
+                                            "launches")] + [("threads", C.c_ulonglong)]
+
+
+fake.host_hip_counts.restype = C.POINTER(Counts)
+fake.host_hip_arg.restype = C.POINTER(C.c_ubyte)
+counts = fake.host_hip_counts().contents
+native.init(0)
+L = native.lib()
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    lib = str(tmp_path_factory.mktemp("host_hip") / "libhost_hip.so")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(rocm, "include"),
+                           os.path.join(HERE, "cpp", "host_hip.cpp"), "-o", lib])
+
+    def go(code):
+        r = subprocess.run([sys.executable, "-c", PRELUDE % (REPO, lib) + code], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return go
+
+
+def test_a_refused_call_does_not_fail_the_next_roadmap(run):
+    run("""
+r = native.Robot(load_robot("fr3"))
+ns = native.Scene(Scene(spheres=np.array([[1, 0, 1, 0.1]], np.float32)))
+q = np.zeros((2, r.dof), np.float32)
+p = C.c_void_p()
+assert L.mp_device_alloc(C.byref(p), 1 << 50) == native.MP_E_NOMEM
+rm = native.Roadmap(r, ns, q[:1], q[1:], samples_per_iteration=8)
+assert L.mp_device_alloc(C.byref(p), 1 << 50) == native.MP_E_NOMEM
+got = rm.read()
+assert got["nv"] == 2
+# a launch that is refused itself is reported
+fake.host_hip_fail(0, 719)
+try:
+    rm.read()
+except native.MPError as e:
+    assert "(-2)" in str(e)
+else:
+    raise AssertionError("the launch failed")
+try:
+    native.Roadmap(r, ns, q[:1], q[1:], samples_per_iteration=8)
+except native.MPError as e:
+    assert "(-2)" in str(e)
+else:
+    raise AssertionError("the launch failed")
+""")
