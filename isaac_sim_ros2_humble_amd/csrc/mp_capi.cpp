@@ -694,9 +694,11 @@ int mp_nn_argmin(const float* d_tree, int n_nodes, int capacity, int dof, const 
         auto mod = mp::get_module({});
         void* args[] = {&d_tree, &n_nodes, &capacity, &dof, &d_q, &nq, &d_idx};
         // two queries per workgroup (the kernel's MP_NN_Q), up to 16 waves (its launch bound) that share
-        // the nodes: one wave per 256 nodes, below which more waves cost more than they save
-        const int waves = std::min(16, std::max(1, (n_nodes + 255) / 256));
-        mp::launch(mod->fn("mp_nn_generic"), (unsigned)((nq + 1) / 2), 64u * waves, stream_of(stream), args, "nn");
+        // the nodes: one wave per 256 nodes, below which more waves cost more than they save.  From 2^21
+        // workgroups on (a launch of 2^32 threads is refused) they take several groups of queries.
+        const int waves = std::min(16, std::max(1, n_nodes / 256 + (n_nodes % 256 ? 1 : 0)));
+        const unsigned groups = std::min(1u << 21, (unsigned)nq / 2 + (unsigned)nq % 2);
+        mp::launch(mod->fn("mp_nn_generic"), groups, 64u * waves, stream_of(stream), args, "nn");
     });
 }
 

@@ -65,3 +65,16 @@ def test_no_nodes_and_no_numbers():
     q = np.zeros((3, 7), np.float32)
     assert np.array_equal(native.nn_argmin(np.zeros((0, 7), np.float32), q), [-1, -1, -1])
     assert np.array_equal(native.nn_argmin(np.full((300, 7), np.nan, np.float32), q), [0x7fffffff] * 3)
+
+
+@pytest.mark.parametrize("n,nq", [(9, (1 << 22) + 5), (4100, (1 << 22) + 2)])
+def test_nearest_nodes_of_more_queries_than_workgroups(n, nq):
+    # coordinates on a grid: distances are whole numbers, exact in float32, with many ties
+    rng = np.random.default_rng(n)
+    tree = rng.integers(-40, 41, (n, 2)).astype(np.float32)
+    at = rng.integers(-45, 46, (nq, 2))
+    side = np.arange(-45, 46)
+    grid = np.stack(np.meshgrid(side, side, indexing="ij"), axis=-1).reshape(-1, 2)
+    want = np.concatenate([np.argmin(((g[:, None, :] - tree[None]) ** 2).sum(2), axis=1) for g in np.array_split(grid, 64)])
+    got = native.nn_argmin(tree, at.astype(np.float32))
+    assert np.array_equal(got, want[(at[:, 0] + 45) * 91 + at[:, 1] + 45])

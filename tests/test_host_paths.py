@@ -73,3 +73,12 @@ except native.MPError as e:
 else:
     raise AssertionError("the launch failed")
 """)
+
+
+@pytest.mark.parametrize("nq", [1, 2, 3, (1 << 22) - 1, (1 << 22) + 1, 9000001, 67000000, (1 << 31) - 1])
+def test_nearest_nodes_of_any_number_of_queries(nq, run):
+    # a launch may hold fewer than 2^32 threads
+    run("""
+for n in (1, 256, 257, 50000, (1 << 31) - 1):
+    assert L.mp_nn_argmin(1 << 20, n, n, 7, 1 << 20, %d, 1 << 20, None) == 0, L.mp_last_error()
+""" % nq)
