@@ -82,3 +82,38 @@ def test_nearest_nodes_of_any_number_of_queries(nq, run):
 for n in (1, 256, 257, 50000, (1 << 31) - 1):
     assert L.mp_nn_argmin(1 << 20, n, n, 7, 1 << 20, %d, 1 << 20, None) == 0, L.mp_last_error()
 """ % nq)
+
+
+def test_a_failed_update_leaves_the_scene_as_it_was(run):
+    # the scene as the check kernel receives it: four counts, then the addresses of its sections
+    run("""
+m = load_robot("fr3")
+r = native.Robot(m)
+rng = np.random.default_rng(0)
+big = workloads.c2_scene(seed=0)
+assert all(c > 2 for c in big.counts)
+small = Scene(spheres=big.spheres[:1], boxes=big.boxes[:2], cylinders=big.cylinders[:1], capsules=big.capsules[:2])
+ns = native.Scene(big)
+fake.host_hip_copy_arg(2, 80)
+
+
+def seen():
+    assert L.mp_check_states(r.h, ns.h, 1 << 20, 64, 1 << 20, None, None) == 0
+    return bytes(fake.host_hip_arg()[:80])
+
+
+before = seen()
+fake.host_hip_fail(719, 0)
+try:
+    ns.update(small)
+except native.MPError as e:
+    assert "(-2)" in str(e)
+else:
+    raise AssertionError("the copy failed")
+fake.host_hip_fail(0, 0)
+assert seen() == before
+ns.update(small)
+assert seen() != before
+ns.update(big)
+assert seen() == before
+""")
