@@ -141,8 +141,9 @@ struct LaunchPlan {
 LaunchPlan plan_launch(int nq, mp_robot* const* robots, const mp_scene* const* scenes, const mp_rrtc_params* params,
                        int default_wave_count);
 
-// The start and goal states of a roadmap (states [ns + ng][dof], loop state [nctl]; host memory that the
-// device maps) into its arrays, one launch.
+// Rows first to first + count - 1 of a roadmap's start and goal states [ns + ng][dof] into its arrays,
+// and the loop state [nctl], one launch.  states (the first of those rows) and state lie in host memory
+// that the device maps.
 struct RoadmapStart {
     const float* states;
     const int* state;
@@ -151,11 +152,12 @@ struct RoadmapStart {
     int* gv[2];
     int* vgroup;
     int* ctl;
-    int ns, ng, dof, vcap, nctl;
+    int ns, first, count, dof, vcap, nctl;
 };
 void roadmap_start(const RoadmapStart& a, hipStream_t s);
-// A roadmap of nv vertices, ne edges and n members laid out as the caller reads it, into host memory
-// that the device maps, one launch.
+// Words first to first + count - 1 of a roadmap as the caller reads it -- vertices, groups, edges, weights,
+// start members, goal members; array i has the words at[i] to at[i + 1] - 1, none when it is not wanted --
+// into host memory that the device maps, one launch.
 struct RoadmapPack {
     const float* node;
     const int* vgroup;
@@ -163,12 +165,9 @@ struct RoadmapPack {
     const int* eb;
     const float* ew;
     const int* gv[2];
-    int nv, ne, n[2], dof, vcap;
-    float* vertices;
-    int* groups;
-    int* edges;
-    float* weights;
-    int* members[2];
+    int dof, vcap;
+    long long at[7], first, count;
+    unsigned* out;
 };
 void roadmap_pack(const RoadmapPack& a, hipStream_t s);
 void roadmap_release_storage();  // frees the kept storage of destroyed roadmaps

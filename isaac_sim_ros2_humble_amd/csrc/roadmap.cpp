@@ -69,6 +69,7 @@ struct Storage {
 };
 constexpr size_t kStateBytes = 256;             // loop state at the head of the host allocation
 constexpr size_t kHostBytes = 256 << 10;        // host allocation of a new roadmap, unless it needs more
+constexpr size_t kHostMost = 1 << 20;           // what does not fit this goes through it in pieces
 constexpr size_t kKeep = 4, kKeepBytes = 8 << 20;  // storage kept: so many, each allocation up to so large
 std::mutex g_mu;                                // guards g_kept
 std::vector<Storage> g_kept;
@@ -251,24 +252,30 @@ int mp_roadmap_create(mp_robot* robot, const mp_scene* scene, const float* start
         int vcap = 4096;
         while (vcap < nv0 + kDepth * 2 * g.k) vcap *= 2;
         try {
-            const size_t state_floats = (size_t)nv0 * dof;
-            take_storage(rm->mem, place(g, nullptr, vcap, 2 * vcap), kStateBytes + state_floats * sizeof(float));
+            const size_t row = (size_t)dof * sizeof(float);
+            take_storage(rm->mem, place(g, nullptr, vcap, 2 * vcap), std::min(kStateBytes + (size_t)nv0 * row, kHostMost));
             place(g, rm->mem.dev, vcap, 2 * vcap);
             rm->mirror_h = reinterpret_cast<int*>(rm->mem.host);
             g.mirror = reinterpret_cast<int*>(rm->mem.host_dev);
-            // the start and goal states: vertices, and the first members of their groups
-            float* states = reinterpret_cast<float*>(rm->mem.host + kStateBytes);
-            std::memcpy(states, starts, (size_t)ns * dof * sizeof(float));
-            std::memcpy(states + (size_t)ns * dof, goals, (size_t)ng * dof * sizeof(float));
             int ctl[kNctl] = {0};
             ctl[NV] = nv0;
             ctl[G1] = ns;
             ctl[G2] = ng;
             ctl[TRAVEL1] = ctl[TRAVEL2] = f2i(max_travel_distance);
             std::memcpy(rm->mirror_h, ctl, sizeof(ctl));
-            mp::roadmap_start({reinterpret_cast<const float*>(rm->mem.host_dev + kStateBytes), g.mirror, g.node,
-                               {g.gq[0], g.gq[1]}, {g.gv[0], g.gv[1]}, g.vgroup, g.ctl, ns, ng, dof, vcap, kNctl},
-                              mp::lib_stream());
+            // the start and goal states: vertices, and the first members of their groups
+            hipStream_t s = mp::lib_stream();
+            const int rows = (int)std::min((size_t)nv0, (rm->mem.host_bytes - kStateBytes) / row);
+            for (int v = 0; v < nv0; v += rows) {
+                const int n = std::min(rows, nv0 - v), n_starts = std::max(0, std::min(n, ns - v));
+                char* const states = rm->mem.host + kStateBytes;
+                if (v > 0) MP_HIP(hipStreamSynchronize(s));  // the rows before have been read
+                if (n_starts > 0) std::memcpy(states, starts + (size_t)v * dof, n_starts * row);
+                if (n > n_starts)
+                    std::memcpy(states + n_starts * row, goals + (size_t)(v + n_starts - ns) * dof, (n - n_starts) * row);
+                mp::roadmap_start({reinterpret_cast<const float*>(rm->mem.host_dev + kStateBytes), g.mirror, g.node,
+                                   {g.gq[0], g.gq[1]}, {g.gv[0], g.gv[1]}, g.vgroup, g.ctl, ns, v, n, dof, vcap, kNctl}, s);
+            }
             mp::Module& mod = *robot->module;
             rm->f_sample = mod.fn("mp_rm_sample_0");
             rm->f_edges = mod.fn("mp_rm_edges_0");
@@ -347,34 +354,37 @@ int mp_roadmap_read(mp_roadmap* rm, float* vertices, int* groups, int* edges, fl
         const RoadmapDevHost& g = rm->g;
         const volatile int* c = rm->mirror_h;
         const size_t nv = (size_t)c[NV], ne = (size_t)c[NE], n1 = (size_t)c[G1], n2 = (size_t)c[G2], dof = (size_t)g.dof;
-        const size_t words[6] = {nv * dof, nv, 2 * ne, ne, n1, n2};
-        size_t at[7] = {kStateBytes};
-        for (int i = 0; i < 6; i++) at[i + 1] = at[i] + words[i] * 4;
-        if (at[6] > rm->mem.host_bytes) {  // the loop state moves along
-            Storage old = rm->mem;
-            rm->mem.host = rm->mem.host_dev = nullptr;
-            try {
-                host_alloc(rm->mem, at[6] + at[6] / 2);
-            } catch (...) {
-                if (rm->mem.host) hipHostFree(rm->mem.host);
-                rm->mem = old;
-                throw;
-            }
-            std::memcpy(rm->mem.host, old.host, kStateBytes);
-            hipHostFree(old.host);
-            rm->mirror_h = reinterpret_cast<int*>(rm->mem.host);
-            rm->g.mirror = reinterpret_cast<int*>(rm->mem.host_dev);
-        }
-        char* const d = rm->mem.host_dev;
-        hipStream_t s = mp::lib_stream();
-        mp::roadmap_pack({g.node, g.vgroup, g.ea, g.eb, g.ew, {g.gv[0], g.gv[1]}, (int)nv, (int)ne, {(int)n1, (int)n2}, g.dof, g.vcap,
-                          (float*)(d + at[0]), (int*)(d + at[1]), (int*)(d + at[2]), (float*)(d + at[3]),
-                          {(int*)(d + at[4]), (int*)(d + at[5])}},
-                         s);
-        MP_HIP(hipStreamSynchronize(s));
         void* const to[6] = {vertices, groups, edges, weights, start_members, goal_members};
-        for (int i = 0; i < 6; i++)
-            if (to[i] && words[i]) std::memcpy(to[i], rm->mem.host + at[i], words[i] * 4);
+        const size_t words[6] = {nv * dof, nv, 2 * ne, ne, n1, n2};
+        mp::RoadmapPack p{g.node, g.vgroup, g.ea, g.eb, g.ew, {g.gv[0], g.gv[1]}, g.dof, g.vcap, {0}, 0, 0, nullptr};
+        for (int i = 0; i < 6; i++) p.at[i + 1] = p.at[i] + (to[i] ? (long long)words[i] : 0);
+        const long long total = p.at[6];
+        if (kStateBytes + (size_t)total * 4 > rm->mem.host_bytes && rm->mem.host_bytes < kHostMost) {
+            Storage more;  // the loop state moves along; without the memory the roadmap goes in smaller pieces
+            try {
+                host_alloc(more, kHostMost);
+                std::memcpy(more.host, rm->mem.host, kStateBytes);
+                std::swap(more.host, rm->mem.host);
+                std::swap(more.host_dev, rm->mem.host_dev);
+                std::swap(more.host_bytes, rm->mem.host_bytes);
+                rm->mirror_h = reinterpret_cast<int*>(rm->mem.host);
+                rm->g.mirror = reinterpret_cast<int*>(rm->mem.host_dev);
+            } catch (const Error&) {
+            }
+            free_storage(more);
+        }
+        const long long room = (long long)(rm->mem.host_bytes - kStateBytes) / 4;
+        const char* const got = rm->mem.host + kStateBytes;
+        p.out = reinterpret_cast<unsigned*>(rm->mem.host_dev + kStateBytes);
+        for (p.first = 0; p.first < total; p.first += room) {
+            p.count = std::min(room, total - p.first);
+            mp::roadmap_pack(p, mp::lib_stream());
+            MP_HIP(hipStreamSynchronize(mp::lib_stream()));
+            for (int i = 0; i < 6; i++) {
+                const long long lo = std::max(p.first, p.at[i]), hi = std::min(p.first + p.count, p.at[i + 1]);
+                if (lo < hi) std::memcpy((char*)to[i] + (lo - p.at[i]) * 4, got + (lo - p.first) * 4, (size_t)(hi - lo) * 4);
+            }
+        }
     });
 }
 

@@ -23,6 +23,7 @@ hipError_t fail_memcpy = hipSuccess, fail_launch = hipSuccess;
 void** last_args = nullptr;  // of the running launch
 unsigned char arg_copy[256];
 int copy_arg = -1, copy_bytes = 0;
+long long host_limit = 1ll << 40;
 
 hipError_t done(hipError_t e) {
     if (e != hipSuccess) last = e;
@@ -53,6 +54,7 @@ void host_hip_copy_arg(int arg, int bytes) {  // keep that argument of the launc
     copy_arg = arg;
     copy_bytes = bytes;
 }
+void host_hip_limit(long long bytes) { host_limit = bytes; }  // of pinned host memory
 const unsigned char* host_hip_arg() { return arg_copy; }
 void host_hip_reset_peak() { counts.host_peak = counts.host_bytes; }
 
@@ -103,6 +105,7 @@ hipError_t hipFree(void* p) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    if (counts.host_bytes + (long long)n > host_limit) return done(hipErrorOutOfMemory);
     *p = std::calloc(n ? n : 1, 1);
     host[*p] = n;
     counts.host_allocs++;

@@ -115,3 +115,27 @@ def test_roadmaps_one_after_another_and_together(fr3, orc_fr3):
     first, second = make(3, 1, 6), make(1, 4, 7)
     finish(second, 1, 4, 7)
     finish(first, 3, 1, 6)
+
+
+def test_large_roadmap_in_pieces(fr3, orc_fr3):
+    """States of some megabytes enter and leave through host memory of one megabyte; any array may be left
+    out of a read."""
+    rng = np.random.default_rng(8)
+    scene = workloads.random_scene(rng, 12, *workloads.workspace(fr3))
+    r, ns = robot(fr3), native.Scene(scene)
+    q = workloads.uniform_configs(fr3, 300001, rng)
+    a, b = 50003, 30011
+    q = q[native.check_states(r, ns, q).astype(bool)][:a + b]
+    assert len(q) == a + b
+    rm = native.Roadmap(r, ns, q[:a], q[a:], samples_per_iteration=64, max_travel_distance=0.7, resolution=0.02, seed=9)
+    rm.iterate()
+    got = rm.read()
+    assert_same(got, oracle.rrg(orc_fr3, oracle.OracleScene(scene), q[:a], q[a:], 64, 0.7, 0.02, 9, 0, max_passes=1, vcap=1 << 18))
+    assert got["nv"] > a + b and got["ne"] > 0
+    names = ("vertices", "groups", "edges", "weights", "start_members", "goal_members")
+    for wanted in [{n} for n in names] + [set(names) - {n} for n in names] + [set()]:
+        out = {n: np.full_like(got[n], -7) for n in wanted}
+        native.check(native.lib().mp_roadmap_read(rm.h, *[native._p(out.get(n)) for n in names]), "mp_roadmap_read")
+        for n in wanted:
+            assert np.array_equal(out[n], got[n]), n
+    rm.close()

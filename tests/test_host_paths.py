@@ -117,3 +117,33 @@ assert seen() != before
 ns.update(big)
 assert seen() == before
 """)
+
+
+def test_pinned_memory_of_large_roadmaps(run):
+    # the host memory that a roadmap pins does not grow with its states, nor with what is read of it
+    run("""
+fake.host_hip_limit.argtypes = [C.c_longlong]
+r = native.Robot(load_robot("fr3"))
+ns = native.Scene(Scene(spheres=np.array([[1, 0, 1, 0.1]], np.float32)))
+n = 200000
+q = np.zeros((n, r.dof), np.float32)
+before = counts.host_bytes
+MOST = 1 << 20
+rm = native.Roadmap(r, ns, q, q, samples_per_iteration=8)
+assert counts.host_bytes - before <= MOST
+fake.host_hip_reset_peak()
+weights = np.zeros(1, np.float32)
+assert L.mp_roadmap_read(rm.h, None, None, None, native._p(weights), None, None) == 0
+groups = np.zeros(2 * n, np.int32)
+assert L.mp_roadmap_read(rm.h, None, native._p(groups), None, None, None, None) == 0
+rm.read()
+assert counts.host_peak - before <= 2 * MOST and counts.host_bytes - before <= MOST
+small = native.Roadmap(r, ns, q[:3], q[:2], samples_per_iteration=8)
+# without a byte more of it, reading goes on in smaller pieces
+big = native.Roadmap(r, ns, q[:5000], q[:4000], samples_per_iteration=8)
+fake.host_hip_limit(counts.host_bytes)
+launched = counts.launches
+big.read()
+assert counts.launches > launched + 1
+small.read()
+""")
