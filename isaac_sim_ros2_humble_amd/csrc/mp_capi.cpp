@@ -58,7 +58,7 @@ int lib_num_cus() { return G.num_cus; }
 unsigned long long* lib_plan_profile() { return G.prof_on ? G.prof : nullptr; }
 unsigned long long* lib_work_counter() { return G.work; }
 
-void launch(hipFunction_t f, unsigned grid, unsigned block, hipStream_t s, void** args, const char* family) {
+void launch(hipFunction_t f, unsigned grid, unsigned block, hipStream_t s, void** args, const char* family, unsigned grid_y) {
     if (grid == 0) return;
     std::pair<hipEvent_t, hipEvent_t> ev{nullptr, nullptr};
     if (family) {
@@ -73,7 +73,7 @@ void launch(hipFunction_t f, unsigned grid, unsigned block, hipStream_t s, void*
         ev = it->second;
     }
     if (ev.first) MP_HIP(hipEventRecord(ev.first, s));
-    MP_HIP(hipModuleLaunchKernel(f, grid, 1, 1, block, 1, 1, 0, s, args, nullptr));
+    MP_HIP(hipModuleLaunchKernel(f, grid, grid_y, 1, block, 1, 1, 0, s, args, nullptr));
     if (ev.second) MP_HIP(hipEventRecord(ev.second, s));
 }
 
@@ -698,11 +698,12 @@ int mp_nn_argmin(const float* d_tree, int n_nodes, int capacity, int dof, const 
         auto mod = mp::get_module({});
         void* args[] = {&d_tree, &n_nodes, &capacity, &dof, &d_q, &nq, &d_idx};
         // two queries per workgroup (the kernel's MP_NN_Q), up to 16 waves (its launch bound) that share
-        // the nodes: one wave per 256 nodes, below which more waves cost more than they save.  From 2^21
-        // workgroups on (a launch of 2^32 threads is refused) they take several groups of queries.
+        // the nodes: one wave per 256 nodes, below which more waves cost more than they save.  Rows of 2^21
+        // workgroups (the kernel's MP_NN_GRID), as 2^32 threads in one dimension are refused.
         const int waves = std::min(16, std::max(1, n_nodes / 256 + (n_nodes % 256 ? 1 : 0)));
-        const unsigned groups = std::min(1u << 21, (unsigned)nq / 2 + (unsigned)nq % 2);
-        mp::launch(mod->fn("mp_nn_generic"), groups, 64u * waves, stream_of(stream), args, "nn");
+        const unsigned groups = (unsigned)nq / 2 + (unsigned)nq % 2, row = 1u << 21;
+        mp::launch(mod->fn("mp_nn_generic"), std::min(groups, row), 64u * waves, stream_of(stream), args, "nn",
+                   (groups + row - 1) / row);
     });
 }
 

@@ -72,7 +72,7 @@ hipStream_t lib_stream();
 int lib_num_cus();
 unsigned long long* lib_plan_profile();  // device counters when the phase profile is on, else null
 unsigned long long* lib_work_counter();  // the algorithmic-flop counter of the check kernels
-void launch(hipFunction_t f, unsigned grid, unsigned block, hipStream_t s, void** args, const char* family);
+void launch(hipFunction_t f, unsigned grid, unsigned block, hipStream_t s, void** args, const char* family, unsigned grid_y = 1);
 SceneDevHost scene_view(const mp_scene* sc);
 void plan_release_workspaces();
 

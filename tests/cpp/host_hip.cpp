@@ -14,7 +14,7 @@ struct Counts {
     long long device_allocs, device_bytes;  // bytes: held now
     long long host_allocs, host_bytes, host_peak;
     long long launches;
-    unsigned long long threads;  // of the last launch
+    unsigned long long workgroups;  // of the last launch
 };
 Counts counts;
 std::map<void*, size_t> device, host;
@@ -31,11 +31,12 @@ hipError_t done(hipError_t e) {
 }
 
 // What a launch may hold: the packet counts threads per dimension in 32 bits.
-hipError_t launch(unsigned long long grid, unsigned long long block, void** args) {
+hipError_t launch(dim3 g, dim3 b, void** args) {
     if (fail_launch != hipSuccess) return done(fail_launch);
-    if (block > 1024 || grid * block > 0xffffffffull) return done(hipErrorInvalidConfiguration);
+    if ((unsigned long long)b.x * b.y * b.z > 1024 || (unsigned long long)g.x * b.x > 0xffffffffull || g.y > 65535 || g.z > 65535)
+        return done(hipErrorInvalidConfiguration);
     counts.launches++;
-    counts.threads = grid * block;
+    counts.workgroups = (unsigned long long)g.x * g.y * g.z;
     if (copy_arg >= 0 && args) std::memcpy(arg_copy, args[copy_arg], (size_t)copy_bytes);
     return hipSuccess;
 }
@@ -137,10 +138,10 @@ hipError_t hipModuleUnload(hipModule_t m) { std::free((void*)m); return hipSucce
 hipError_t hipModuleGetFunction(hipFunction_t* f, hipModule_t, const char*) { *f = (hipFunction_t)&counts; return hipSuccess; }
 hipError_t hipModuleLaunchKernel(hipFunction_t, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned by, unsigned bz,
                                  unsigned, hipStream_t, void** args, void**) {
-    return launch((unsigned long long)gx * gy * gz, (unsigned long long)bx * by * bz, args);
+    return launch(dim3(gx, gy, gz), dim3(bx, by, bz), args);
 }
 hipError_t hipLaunchKernel(const void*, dim3 g, dim3 b, void** args, size_t, hipStream_t) {
-    return launch((unsigned long long)g.x * g.y * g.z, (unsigned long long)b.x * b.y * b.z, args);
+    return launch(g, b, args);
 }
 
 }  // extern "C"

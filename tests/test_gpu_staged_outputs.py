@@ -67,8 +67,8 @@ def test_no_nodes_and_no_numbers():
     assert np.array_equal(native.nn_argmin(np.full((300, 7), np.nan, np.float32), q), [0x7fffffff] * 3)
 
 
-@pytest.mark.parametrize("n,nq", [(9, (1 << 22) + 5), (4100, (1 << 22) + 2)])
-def test_nearest_nodes_of_more_queries_than_workgroups(n, nq):
+@pytest.mark.parametrize("n,nq", [(9, (1 << 22) + 5), (4100, (1 << 22) + 2), (4100, 9000001)])
+def test_nearest_nodes_of_millions_of_queries(n, nq):
     # coordinates on a grid: distances are whole numbers, exact in float32, with many ties
     rng = np.random.default_rng(n)
     tree = rng.integers(-40, 41, (n, 2)).astype(np.float32)

@@ -23,7 +23,7 @@ from isaac_sim_ros2_humble_amd.scene import Scene
 
 class Counts(C.Structure):
     _fields_ = [(f, C.c_longlong) for f in ("device_allocs", "device_bytes", "host_allocs", "host_bytes", "host_peak",
-                                            "launches")] + [("threads", C.c_ulonglong)]
+                                            "launches")] + [("workgroups", C.c_ulonglong)]
 
 
 fake.host_hip_counts.restype = C.POINTER(Counts)
@@ -77,11 +77,12 @@ else:
 
 @pytest.mark.parametrize("nq", [1, 2, 3, (1 << 22) - 1, (1 << 22) + 1, 9000001, 67000000, (1 << 31) - 1])
 def test_nearest_nodes_of_any_number_of_queries(nq, run):
-    # a launch may hold fewer than 2^32 threads
+    # a launch may hold fewer than 2^32 threads per dimension; two queries per workgroup
     run("""
 for n in (1, 256, 257, 50000, (1 << 31) - 1):
     assert L.mp_nn_argmin(1 << 20, n, n, 7, 1 << 20, %d, 1 << 20, None) == 0, L.mp_last_error()
-""" % nq)
+    assert counts.workgroups >= -(-%d // 2)
+""" % (nq, nq))
 
 
 def test_a_failed_update_leaves_the_scene_as_it_was(run):
