@@ -74,6 +74,10 @@ constexpr size_t kKeep = 4, kKeepBytes = 8 << 20;  // storage kept: so many, eac
 std::mutex g_mu;                                // guards g_kept
 std::vector<Storage> g_kept;
 
+bool smaller(const Storage& a, const Storage& b) {
+    return a.dev_bytes != b.dev_bytes ? a.dev_bytes < b.dev_bytes : a.host_bytes < b.host_bytes;
+}
+
 void host_alloc(Storage& st, size_t bytes) {
     MP_HIP(hipHostMalloc((void**)&st.host, bytes, hipHostMallocMapped | hipHostMallocCoherent));
     st.host_bytes = bytes;
@@ -88,18 +92,23 @@ void free_storage(Storage& st) {
     st = Storage();
 }
 
-// Kept storage with room for the sizes, else new.  `st` is the caller's to free also when this throws.
+// The smallest kept storage with room for the sizes, else new.  `st` is the caller's to free also when
+// this throws.
 void take_storage(Storage& st, size_t dev_bytes, size_t host_bytes) {
     int device = 0;
     MP_HIP(hipGetDevice(&device));
     {
         std::lock_guard<std::mutex> g(g_mu);
-        for (size_t i = 0; i < g_kept.size(); i++)
-            if (g_kept[i].device == device && g_kept[i].dev_bytes >= dev_bytes && g_kept[i].host_bytes >= host_bytes) {
-                st = g_kept[i];
-                g_kept.erase(g_kept.begin() + (long)i);
-                return;
-            }
+        auto best = g_kept.end();
+        for (auto it = g_kept.begin(); it != g_kept.end(); ++it)
+            if (it->device == device && it->dev_bytes >= dev_bytes && it->host_bytes >= host_bytes &&
+                (best == g_kept.end() || smaller(*it, *best)))
+                best = it;
+        if (best != g_kept.end()) {
+            st = *best;
+            g_kept.erase(best);
+            return;
+        }
     }
     st.device = device;
     MP_HIP(hipMalloc((void**)&st.dev, dev_bytes));
@@ -108,14 +117,17 @@ void take_storage(Storage& st, size_t dev_bytes, size_t host_bytes) {
     for (auto& e : st.ev) MP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 }
 
-// Keeps whole storage that no work uses any more (the caller has waited for the stream) or frees it.
+// Keeps whole storage that no work uses any more (the caller has waited for the stream), in the place of
+// the smallest kept when there are enough, or frees it.
 void give_back(Storage& st) {
     if (st.dev && st.host_dev && st.ev[kDepth - 1] && st.dev_bytes <= kKeepBytes && st.host_bytes <= kKeepBytes) {
         std::lock_guard<std::mutex> g(g_mu);
         if (g_kept.size() < kKeep) {
             g_kept.push_back(st);
             st = Storage();
-            return;
+        } else {
+            auto least = std::min_element(g_kept.begin(), g_kept.end(), smaller);
+            if (smaller(*least, st)) std::swap(*least, st);
         }
     }
     free_storage(st);

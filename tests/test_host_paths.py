@@ -148,3 +148,46 @@ big.read()
 assert counts.launches > launched + 1
 small.read()
 """)
+
+
+def test_kept_roadmap_storage_follows_the_roadmaps_in_use(run):
+    # four roadmaps' storage is kept: the largest that were given back, the smallest that fits handed out
+    run("""
+r = native.Robot(load_robot("fr3"))
+ns = native.Scene(Scene(spheres=np.array([[1, 0, 1, 0.1]], np.float32)))
+q = np.zeros((70000, r.dof), np.float32)
+
+
+def make(n):
+    return native.Roadmap(r, ns, q[:n], q[:1], samples_per_iteration=8)
+
+
+def allocates(f):
+    before = counts.device_allocs
+    f()
+    return counts.device_allocs - before
+
+
+for rm in [make(10) for _ in range(4)]:
+    rm.close()
+assert allocates(lambda: make(10).close()) == 0
+# a larger one takes the place of a small one, also where four small ones are kept
+assert allocates(lambda: make(6000).close()) == 1
+assert allocates(lambda: make(6000).close()) == 0
+for _ in range(3):  # small and large by turns, more than are kept
+    assert allocates(lambda: make(10).close()) == 0
+    assert allocates(lambda: make(6000).close()) == 0
+# a small one leaves the large one alone
+small = make(10)
+assert allocates(lambda: make(6000).close()) == 0
+small.close()
+# what is too large to keep is freed
+held = counts.device_bytes
+assert allocates(lambda: make(70000).close()) == 1
+assert counts.device_bytes == held
+# four at once of the larger size: the small ones are gone, and a small roadmap takes a larger storage
+for rm in [make(6000) for _ in range(4)]:
+    rm.close()
+assert allocates(lambda: make(10).close()) == 0
+L.mp_shutdown()
+""")
