@@ -2,6 +2,8 @@
 64-obstacle chunks, batches at the edges of the states-per-wave split, a NaN state among free ones,
 and a scene that shrinks.  Verdicts, costs and motions equal the oracle's bit for bit (the cull only
 skips what cannot touch, so there is no tolerance)."""
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -101,3 +103,91 @@ def test_lanes_walk_their_own_obstacles(name, kind, count, robots, request):
     vo, _, _, _ = oracle.check(request.getfixturevalue("orc_" + name), oracle.OracleScene(scene), q, nthreads=8)
     assert 0 < vo.sum() < len(vo)
     assert np.array_equal(native.check_states(robots[name], native.Scene(scene), q), vo)
+
+
+def _reachable(model, kind, count, seed):
+    """`count` obstacles of a kind (or all four) among the arm's links."""
+    rng = np.random.default_rng(seed)
+
+    def pos():
+        return rng.uniform([0.4, -0.8, 0.2], [1.0, 0.8, 1.3])
+    make = {"boxes": lambda: box_record(pos(), random_rotation(rng), rng.uniform(0.01, 0.06, 3)),
+            "cylinders": lambda: cylinder_record(pos(), random_rotation(rng), rng.uniform(0.01, 0.06), rng.uniform(0.05, 0.2)),
+            "capsules": lambda: capsule_record(pos(), random_rotation(rng), rng.uniform(0.01, 0.06), rng.uniform(0.05, 0.2)),
+            "spheres": lambda: np.append(pos(), rng.uniform(0.01, 0.07))}
+    kinds = list(make) if kind == "mixed" else [kind]
+    scene = Scene(**{k: np.array([make[k]() for _ in range(len(range(i, count, len(kinds))))], np.float32)
+                     for i, k in enumerate(kinds)})
+    assert scene.num_obstacles == count
+    return scene
+
+
+def _path(model, n, seed, step=0.005):
+    """States along straight lines between random configurations, `step` rad apart."""
+    knots = workloads.uniform_configs(model, 4 + int(n * step / 2.0) * 2, np.random.default_rng(seed)).astype(np.float64)
+    at = np.concatenate([[0.0], np.cumsum(np.linalg.norm(np.diff(knots, axis=0), axis=1))])
+    s = np.arange(n) * step
+    assert s[-1] < at[-1]
+    return np.stack([np.interp(s, at, knots[:, j]) for j in range(model.dof)], axis=1).astype(np.float32)
+
+
+def _states(model, form, n, seed):
+    """Unrelated states, states along a path, waves of the one beside waves of the other, or both in
+    every wave.  The waves of these batches hold 16, 32 or 64 states."""
+    spread, path = workloads.uniform_configs(model, n, np.random.default_rng(seed)), _path(model, n, seed)
+    run = {"scattered": 1 << 30, "path": 0, "waves": 64, "within": 11}[form]
+    return np.where((np.arange(n) // run % 2 == 0)[:, None], spread, path) if run else path
+
+
+def _oracle_rows(orc, osc, q):
+    with ThreadPoolExecutor(8) as ex:
+        return np.concatenate(list(ex.map(lambda p: oracle.constraint_costs(orc, osc, p), np.array_split(q, 32))), axis=1)
+
+
+@pytest.mark.parametrize("form,name,kind,count,n", [
+    ("scattered", "fr3", "boxes", 31, 20001), ("scattered", "fetch", "boxes", 65, 17003), ("scattered", "fetch", "cylinders", 33, 20001),
+    ("scattered", "fr3", "cylinders", 65, 33001), ("scattered", "fr3", "capsules", 32, 20001), ("scattered", "fetch", "capsules", 66, 17003),
+    ("scattered", "fetch", "spheres", 64, 20001), ("scattered", "fr3", "spheres", 97, 66001), ("scattered", "fr3", "mixed", 130, 40003),
+    ("scattered", "fetch", "mixed", 97, 40003), ("path", "fr3", "mixed", 97, 70003), ("path", "fetch", "mixed", 130, 17003),
+    ("path", "fetch", "boxes", 65, 34001), ("path", "fr3", "spheres", 33, 17003), ("waves", "fr3", "mixed", 130, 70003),
+    ("waves", "fetch", "mixed", 97, 34001), ("within", "fr3", "mixed", 65, 34001), ("within", "fetch", "mixed", 130, 17003),
+    ("scattered", "fr3", "mixed", 0, 17003), ("path", "fetch", "mixed", 1, 17003)])
+def test_large_batches_of_either_form(form, name, kind, count, n, robots, request):
+    # verdicts, centres, total costs and every constraint's row of the launches whose waves choose between
+    # taking their near obstacles one by one and letting each lane walk its own
+    m = request.getfixturevalue(name)
+    orc = request.getfixturevalue("orc_" + name)
+    scene = _reachable(m, kind, count, seed=count + 2)
+    q = _states(m, form, n, seed=n + count)
+    ns, osc = native.Scene(scene), oracle.OracleScene(scene)
+    vo, co, centres, _ = oracle.check(orc, osc, q, want_cost=True, want_centres=True, nthreads=8)
+    rows = _oracle_rows(orc, osc, q)
+    assert 0 < vo.sum() < n
+    assert all((r > 0).any() for r, c in zip(rows, scene.counts) if c > 1)
+    v, c = native.check_states(robots[name], ns, q, want_centres=True)
+    assert np.array_equal(v, vo) and np.array_equal(c, centres)
+    assert np.array_equal(native.check_states(robots[name], ns, q), vo)
+    cost, vc = native.state_costs(robots[name], ns, q)
+    assert np.array_equal(cost, co) and np.array_equal(vc, vo)
+    parts, total, vp = native.constraint_costs(robots[name], ns, q)
+    assert np.array_equal(parts, rows) and np.array_equal(total, co) and np.array_equal(vp, vo)
+
+
+@pytest.mark.parametrize("form,name", [("scattered", "fr3"), ("path", "fr3"), ("scattered", "fetch"), ("path", "fetch")])
+def test_costs_beside_nan_states(form, name, robots, request):
+    # the lanes that the waves' balls are centred on, and others, hold NaN or infinite states
+    m = request.getfixturevalue(name)
+    orc = request.getfixturevalue("orc_" + name)
+    scene = _reachable(m, "mixed", 70, seed=12)
+    q = _states(m, form, 70001, seed=13)
+    q[16::128] = np.nan
+    q[48::192, 3] = np.inf
+    q[5::100, 0] = -np.inf
+    q[7::90, 5] = np.nan
+    keep = np.isfinite(q).all(axis=1)
+    ns, osc = native.Scene(scene), oracle.OracleScene(scene)
+    vo, co, _, _ = oracle.check(orc, osc, q[keep], want_cost=True, nthreads=8)
+    assert np.array_equal(native.check_states(robots[name], ns, q)[keep], vo)
+    parts, total, v = native.constraint_costs(robots[name], ns, q)
+    assert np.array_equal(parts[:, keep], _oracle_rows(orc, osc, q[keep]))
+    assert np.array_equal(total[keep], co) and np.array_equal(v[keep], vo)
