@@ -272,8 +272,9 @@ std::vector<SphereLink> sphere_links(const RobotModel& m) {
 constexpr int kXform = 18, kSelf = 9, kSph = 11, kBox = 34, kCyl = 35, kCap = 28;
 constexpr int kCentreChunk = 16;  // spheres per staged chunk; the LDS row is MP_CENTRE_ROW floats
 constexpr int kPoseChunk = 2;     // links per staged chunk (128 bytes per state); the LDS row is MP_POSE_ROW floats
-// LDS of the FK kernel's tile: whole rows of centres for as many states of a wave as fit.  40 KB keep
-// four one-wave workgroups on a CU, enough to cover the stores' latency with the next states' FK.
+// LDS of the FK kernel's tile: whole rows of centres for as many states of a wave (a power of two) as fit
+// 48 KB.  Three one-wave workgroups fit a CU (FR3 46.9 KB, Fetch 42.3 KB of 160), enough to reach the rate of
+// a large copy.
 constexpr int kCentreTileFloats = 12 * 1024;
 
 }  // namespace
@@ -752,10 +753,10 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     while (crows > 4 && crows * 3 * m.S > kCentreTileFloats) crows /= 2;
     o << "    static constexpr int CROWS = " << crows << ";\n";
     o << "    // out: the wave's first configuration; live: its configurations below n; tile: the wave's\n"
-         "    // LDS tile of MP_WAVE x MP_CENTRE_ROW floats\n"
-         "    static __device__ __forceinline__ void write_centres_staged(const float* F, float* out, int live, float* tile) {\n"
+         "    // LDS tile of MP_WAVE x MP_CENTRE_ROW floats; at: the lane's configuration among them\n"
+         "    static __device__ __forceinline__ void write_centres_staged(const float* F, float* out, int live, float* tile, int at) {\n"
          "        const int lane = threadIdx.x & (MP_WAVE - 1);\n"
-         "        float* row = tile + lane * MP_CENTRE_ROW;\n"
+         "        float* row = tile + at * MP_CENTRE_ROW;\n"
       << staged_body << "    }\n";
     o << "    template <int MODE>\n    static __device__ __forceinline__ bool self_hit(const float* F, bool h, u64 mask, unsigned& work, const Team& T) {\n"
          "        u64 live = mp_live<MODE>(__ballot(h), mask);\n"
@@ -924,13 +925,13 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     int last = NL - 1;
     auto fixed = [&](int k) { return FV[k][9].k && FV[k][10].k && FV[k][11].k && FV[k][0].k; };
     while (last >= 0 && fixed(last)) last--;
-    o << "    static __device__ __forceinline__ bool scattered(const float* F, u64 live) {\n";
+    o << "    static __device__ __forceinline__ bool scattered(const float* F, u64 live, float far) {\n";
     if (last >= 0) {
         Emitter X;
         V b[3];
         link_centre(X, last, b);
         const std::string at = X.ref(b[0]) + ", " + X.ref(b[1]) + ", " + X.ref(b[2]);
-        o << X.os.str() << "        return mp_scattered(mp_half_balls(" << at << ", live));\n    }\n";
+        o << X.os.str() << "        return mp_scattered(mp_half_balls(" << at << ", live), far);\n    }\n";
     } else {
         o << "        return false;\n    }\n";
     }

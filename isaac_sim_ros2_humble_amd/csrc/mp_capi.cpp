@@ -592,20 +592,32 @@ int mp_scene_destroy(mp_scene* sc) {
 
 // ---------------------------------------------------------------------------------------- kernels
 namespace {
-// States per wave of the check and cost kernels: 64 once the launch fills the chip with them (two
-// waves on each of a CU's four SIMDs, what the kernels' registers allow), else the power of two that
-// still makes that many waves.
-int states_per_wave(int64_t n) {
-    const int64_t waves = (int64_t)std::max(G.num_cus, 1) * 8;
-    int c = 64;
-    while (c > 1 && n <= waves * (c / 2)) c /= 2;
-    return c;
+int num_obstacles(const mp_scene* s) { return s->ns + s->nb + s->nc + s->ncap; }
+// States per wave of the check and cost kernels (1 to 64).  A wave's vector instructions keep its SIMD
+// busy by themselves, so a second wave on a SIMD takes as long again unless it has less to do than one wave
+// with the states of both: unrelated states among many obstacles, not neighbouring ones, which share
+// their near obstacles, nor few obstacles.  And every further CU has the kernel's code to fetch.  24,001 FR3
+// states 0.005 rad apart, 20 obstacles, at 64 / 32 / 16 / 8 / 4 states a wave: 19 / 20 / 28 / 52 / 85 us (24 us with 64 in
+// the kernels before the near obstacles by lanes); 2,049 unrelated ones 58 / 52 / 47 / 41 / 37 us.  So four waves
+// on a CU from 32 obstacles on, three from 16, and two below.  States 0.005 rad apart (unrelated ones in
+// brackets): 1,500 FR3 states with 5 obstacles: two 16 us (24), four 19 (21), eight 28 (28); 6,001 with 200:
+// four 25 (186), eight 32 (188).
+int states_per_wave(int64_t n, const mp_scene* s) {
+    const int64_t waves = (int64_t)std::max(G.num_cus, 1) * std::min(4, 2 + num_obstacles(s) / 16);
+    return (int)std::min<int64_t>(64, std::max<int64_t>(1, (n + waves - 1) / waves));
 }
-// Scattered states are worth the kernels that look for them (more registers, a test per wave) only where a
-// wave holds many of them.  FR3: 257 random states (one per wave) 21.7 us without, 24.8 with; a million
-// (64 per wave) 1,128 and 711 us.
-const char* check_kernel(int per_wave) { return per_wave >= 16 ? "mp_check_each_0" : "mp_check_0"; }
-const char* cost_kernel(int per_wave) { return per_wave >= 16 ? "mp_cost_each_0" : "mp_cost_0"; }
+// The kernels whose waves look whether their states are scattered (more registers, some of them spilled, and
+// a test per wave) where waves hold many states and obstacles abound; the kernels without elsewhere.  Unrelated
+// states, without and with, verdicts: 34,001 FR3 states with 5 / 20 / 64 obstacles 38 and 46, 61 and 46, 122 and 67 us, 9,001
+// 32 and 40, 49 and 41, 92 and 57; Fetch 43 and 53, 58 and 56, 68 and 53.  Costs: 34,001 FR3 states 52 and 68, 70 and
+// 72, 193 and 132; Fetch 94 and 106, 107 and 117, 213 and 216 (200 obstacles: 241 and 225).  States 0.005 rad
+// apart pay 2 to 4 us for the test and the registers.
+const char* check_kernel(int per_wave, const mp_scene* s) {
+    return per_wave >= 16 && num_obstacles(s) >= 16 ? "mp_check_each_0" : "mp_check_0";
+}
+const char* cost_kernel(int per_wave, const mp_scene* s) {
+    return per_wave >= 16 && num_obstacles(s) >= 32 ? "mp_cost_each_0" : "mp_cost_0";
+}
 unsigned state_blocks(int64_t n, int per_wave) { return (unsigned)((n + 4 * per_wave - 1) / (4 * per_wave)); }
 }  // namespace
 
@@ -639,9 +651,9 @@ int mp_check_states(const mp_robot* robot, const mp_scene* scene, const float* d
         if (n == 0) return;
         long long nn = n;
         mp::SceneDevHost sv = mp::scene_view(scene);
-        int per_wave = states_per_wave(n);
+        int per_wave = states_per_wave(n, scene);
         void* args[] = {&d_q, &nn, &sv, &d_verdict, &d_centres, &G.work, &per_wave};
-        mp::launch(robot->module->fn(check_kernel(per_wave)), state_blocks(n, per_wave), 256, stream_of(stream), args, "check");
+        mp::launch(robot->module->fn(check_kernel(per_wave, scene)), state_blocks(n, per_wave), 256, stream_of(stream), args, "check");
     });
 }
 
@@ -654,9 +666,9 @@ int mp_state_costs(const mp_robot* robot, const mp_scene* scene, const float* d_
         long long nn = n;
         mp::SceneDevHost sv = mp::scene_view(scene);
         float* d_parts = nullptr;
-        int per_wave = states_per_wave(n);
+        int per_wave = states_per_wave(n, scene);
         void* args[] = {&d_q, &nn, &sv, &d_cost, &d_verdict, &d_parts, &G.work, &per_wave};
-        mp::launch(robot->module->fn(cost_kernel(per_wave)), state_blocks(n, per_wave), 256, stream_of(stream), args, "cost");
+        mp::launch(robot->module->fn(cost_kernel(per_wave, scene)), state_blocks(n, per_wave), 256, stream_of(stream), args, "cost");
     });
 }
 
@@ -668,9 +680,9 @@ int mp_constraint_costs(const mp_robot* robot, const mp_scene* scene, const floa
         if (n == 0) return;
         long long nn = n;
         mp::SceneDevHost sv = mp::scene_view(scene);
-        int per_wave = states_per_wave(n);
+        int per_wave = states_per_wave(n, scene);
         void* args[] = {&d_q, &nn, &sv, &d_cost, &d_verdict, &d_parts, &G.work, &per_wave};
-        mp::launch(robot->module->fn(cost_kernel(per_wave)), state_blocks(n, per_wave), 256, stream_of(stream), args, "cost");
+        mp::launch(robot->module->fn(cost_kernel(per_wave, scene)), state_blocks(n, per_wave), 256, stream_of(stream), args, "cost");
     });
 }
 

@@ -191,3 +191,28 @@ def test_costs_beside_nan_states(form, name, robots, request):
     parts, total, v = native.constraint_costs(robots[name], ns, q)
     assert np.array_equal(parts[:, keep], _oracle_rows(orc, osc, q[keep]))
     assert np.array_equal(total[keep], co) and np.array_equal(v[keep], vo)
+
+
+@pytest.mark.parametrize("name,count,n", [
+    ("fr3", 5, 511), ("fr3", 5, 513), ("fetch", 5, 1025), ("fr3", 20, 2305), ("fetch", 20, 5377), ("fr3", 33, 7001), ("fetch", 33, 16385),
+    ("fr3", 12, 16383), ("fr3", 130, 31749), ("fetch", 15, 32257), ("fr3", 15, 32768), ("fr3", 15, 32769)])
+@pytest.mark.parametrize("form", ["scattered", "path"])
+def test_any_number_of_states_per_wave(form, name, count, n, robots, request):
+    # 1, 2, 3, 4, 7, 16, 17, 32, 63 and 64 states a wave, the last wave's run cut short: centres into a guarded
+    # buffer, verdicts, every constraint's row
+    m = request.getfixturevalue(name)
+    orc = request.getfixturevalue("orc_" + name)
+    scene = _reachable(m, "mixed", count, seed=count + 3)
+    q = _states(m, form, n, seed=n)
+    ns, osc = native.Scene(scene), oracle.OracleScene(scene)
+    vo, co, centres, _ = oracle.check(orc, osc, q, want_cost=True, want_centres=True, nthreads=8)
+    guard = np.float32(-77.25)
+    dq = native.DeviceBuffer.from_array(q)
+    dc = native.DeviceBuffer.from_array(np.full(n * m.S * 3 + 8, guard, np.float32))
+    dv = native.DeviceBuffer.from_array(np.full(n + 8, 9, np.uint8))
+    native.check(native.lib().mp_check_states(robots[name].h, ns.h, dq.ptr, n, dv.ptr + 3, dc.ptr + 4, None), "mp_check_states")
+    v, c = dv.to_array(np.uint8, (n + 8,)), dc.to_array(np.float32, (n * m.S * 3 + 8,))
+    assert np.array_equal(v[3:n + 3], vo) and (v[:3] == 9).all() and (v[n + 3:] == 9).all()
+    assert np.array_equal(c[1:-7].reshape(n, m.S, 3), centres) and c[0] == guard and (c[-7:] == guard).all()
+    parts, total, vp = native.constraint_costs(robots[name], ns, q)
+    assert np.array_equal(total, co) and np.array_equal(vp, vo) and np.array_equal(parts, _oracle_rows(orc, osc, q))

@@ -191,3 +191,24 @@ for rm in [make(6000) for _ in range(4)]:
 assert allocates(lambda: make(10).close()) == 0
 L.mp_shutdown()
 """)
+
+
+@pytest.mark.parametrize("kind,counts", [("check", (5, 2)), ("check", (20, 3)), ("check", (32, 4)), ("check", (200, 4)),
+                                         ("cost", (5, 2)), ("cost", (200, 4))])
+def test_waves_of_small_batches(kind, counts, run):
+    # one wave a SIMD at most, fewer where there are few obstacles, until waves are full: four waves per
+    # workgroup, 256 CUs
+    run("""
+obstacles, per_cu = %r
+r = native.Robot(load_robot("fr3"))
+ns = native.Scene(Scene(spheres=np.ones((obstacles, 4), np.float32)))
+for n in (1, 2, 255, 511, 512, 513, 1025, 1537, 2049, 4099, 6001, 12001, 16385, 24001, 32767, 32768, 32769, 65537, 1 << 20):
+    if %r == "check":
+        assert L.mp_check_states(r.h, ns.h, 1 << 20, n, 1 << 20, None, None) == 0
+    else:
+        assert L.mp_state_costs(r.h, ns.h, 1 << 20, n, 1 << 20, 1 << 20, None) == 0
+    waves = 256 * per_cu
+    per_wave = min(64, -(-n // waves))
+    assert counts.workgroups == -(-n // (4 * per_wave)), n
+    assert per_wave == 64 or counts.workgroups * 4 < waves + 4
+""" % (counts, kind))
