@@ -591,8 +591,8 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     }
     // The link frames made opaque at the head of each near obstacle's block: otherwise the sphere
     // centres, which do not change from obstacle to obstacle, are moved out of the loop, far more of
-    // them than there are registers (FR3's check kernel 258 -> 212 VGPRs, two waves per SIMD again;
-    // mp_plan 383 -> 308)
+    // them than there are registers (FR3 without and with: mp_check 250 and 177 VGPRs, mp_plan 384 and 282;
+    // registers spilled by mp_check_each 61 and 7, mp_cost_each 180 and 10, mp_edges 40 and 0)
     std::string pin;
     for (int k = 0; k < NL; k++)
         for (int e = 0; e < 12; e++)
@@ -806,8 +806,10 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     // verdict's settled lanes leave; the costs take down the obstacles in contact (bits of touch) and then
     // evaluate those in index order, the others' terms being exact zeros.  work counts what each lane did.
     // Bound by the sphere tests' arithmetic and the gathers of the lanes' own records; a function of its
-    // own, as sharing the link masks with the other form spilled 42 registers (730 against 711 us for a
-    // million random FR3 states; the figures of the choice stand at mp_scattered).
+    // own, as sharing the link masks with the other form spilled 42 registers of FR3's kernel (730 against 711
+    // us for a million random FR3 states; the figures of the choice stand at mp_scattered).  The kernels that
+    // hold both forms still spill some of their 256 registers: checks 7 (FR3) and 40 (Fetch), costs 10 and 22,
+    // 32 to 164 bytes of scratch a lane.
     const int row_of[4] = {1, 0, 3, 2};  // costs: box, sphere, capsule, cylinder
     auto each_lane = [&](bool cost) {
         const char* kind_name[4] = {"box", "sph", "cap", "cyl"};
