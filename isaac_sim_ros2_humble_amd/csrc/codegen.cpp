@@ -400,7 +400,7 @@ std::string robot_struct_source(const RobotModel& m, const std::string& sname) {
     };
     auto named = [&](Emitter& X, const V& v) -> std::string { return X.ref(v); };
 
-    std::vector<float> rad(m.sphere_r.begin(), m.sphere_r.end()), boxte(m.S);
+    std::vector<float> boxte(m.S);
     for (int s = 0; s < m.S; s++) boxte[s] = std::min(m.sphere_r[s] * m.sphere_r[s], sqrt_threshold(m.sphere_r[s]));
 
     // ---------------------------------------------------------------- centres output

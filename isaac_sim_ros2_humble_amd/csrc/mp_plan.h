@@ -5,7 +5,6 @@
 
 #include "mp_internal.h"
 
-#define MP_SPH_W_H 4
 #define MP_BOX_W_H 24
 #define MP_CYL_W_H 20
 #define MP_CAP_W_H 12
